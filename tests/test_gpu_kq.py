@@ -1,0 +1,64 @@
+"""k-qubit unitaries on the matrix cores against the oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from gpu_util import rand_state, rand_unitary, to_gpu, to_np
+from oracle import statevector as O
+
+pytestmark = pytest.mark.gpu
+
+# (n, qubits): the smallest tile of each k and one bit below it (general
+# kernel), targets lowest, highest, interleaved and in descending order, chunks
+# and row blocks of k >= 7, several tiles per work-group (19 qubits at k = 4)
+CASES = [
+    (3, [2, 0, 1]), (11, [0, 5, 10]), (12, [11, 10, 9]), (12, [0, 1, 2]),
+    (11, [3, 1, 9, 4]), (12, [3, 1, 9, 4]), (12, [8, 9, 10, 11]), (19, [0, 18, 7, 3]),
+    (12, [11, 0, 6, 3, 9]), (13, [4, 3, 2, 1, 0]), (11, [10, 8, 6, 4, 2]),
+    (12, [0, 2, 4, 6, 8, 10]), (13, [12, 11, 10, 9, 8, 7]), (14, [5, 0, 13, 2, 9, 1]),
+    (12, [0, 1, 2, 3, 4, 5, 6]), (13, [12, 1, 3, 5, 7, 9, 11]), (14, [0, 13, 1, 12, 2, 11, 3, 10]),
+    (15, [14, 0, 2, 4, 6, 8, 10, 12, 13]), (16, [15, 3, 9, 0, 12, 6, 1, 7, 10, 4]),
+]
+
+
+@pytest.mark.parametrize("n,qubits", CASES)
+@pytest.mark.parametrize("offset", [0, 1])  # 1: a state at 8-byte alignment (general kernel)
+def test_kq_against_oracle(n, qubits, offset):
+    import torch
+
+    from tyxonq_amd import kernels as K
+
+    rng = np.random.default_rng(100 * n + len(qubits))
+    v, U = rand_state(rng, n), rand_unitary(rng, 1 << len(qubits))
+    buf = torch.zeros((1 << n) + offset, dtype=torch.complex64, device="cuda")
+    src = buf[offset:]
+    src.copy_(to_gpu(v))
+    out = to_np(K.apply_kqubit_unitary(src, U, qubits, n))
+    ref = O.apply_kqubit(to_np(src), U, qubits, n)
+    # unit-norm rows: 2^(k+1) FP32 products and sums of random sign, 2^-24 each
+    tol = 4 * 2.0 ** -24 * np.sqrt(2.0 ** len(qubits))
+    assert np.linalg.norm(out - ref) <= tol * np.linalg.norm(ref)
+    np.testing.assert_array_equal(to_np(src), to_np(to_gpu(v)))
+
+
+def test_kq_calls_in_flight_on_two_streams():
+    """The tables of a call are staged until its kernel has run."""
+    import torch
+
+    from tyxonq_amd import kernels as K
+
+    n, rng = 14, np.random.default_rng(3)
+    v = to_gpu(rand_state(rng, n))
+    Us = [rand_unitary(rng, 64) for _ in range(8)]
+    qs = [[int(q) for q in rng.choice(n, 6, replace=False)] for _ in Us]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    outs = []
+    for i, (U, q) in enumerate(zip(Us, qs)):
+        with torch.cuda.stream(streams[i % 2]):
+            outs.append(K.apply_kqubit_unitary(v, U, q, n))
+    torch.cuda.synchronize()
+    for U, q, out in zip(Us, qs, outs):
+        ref = O.apply_kqubit(to_np(v), U, q, n)
+        assert np.linalg.norm(to_np(out) - ref) <= 4 * 2.0 ** -24 * 8 * np.linalg.norm(ref)

@@ -1,5 +1,6 @@
 // tqsv_abi.cpp - error state, single-op entry points and plan management of
 // the libtqsv C ABI (declared in include/tqsv.h).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -32,6 +33,81 @@ int scratch(size_t ndoubles, double** out) {
     g_scratch.cap = ndoubles;
   }
   *out = g_scratch.d;
+  return 0;
+}
+
+// Host-to-device staging of per-call tables: two slots per thread, each a
+// page-locked buffer, its device copy and the event after the last kernel that
+// reads it.  A slot is taken again only when that event has passed, so calls
+// need no stream synchronisation, on whatever streams the thread uses.  Slots
+// grow to the largest call (8 MiB for a 10-qubit matrix) and go with the thread.
+struct Upload {
+  unsigned char* h = nullptr;
+  unsigned char* d = nullptr;
+  size_t cap = 0;
+  hipEvent_t ev = nullptr;
+  int dev = -1;
+  bool busy = false;
+  void drop() {
+    if (busy) (void)hipEventSynchronize(ev);
+    if (ev) (void)hipEventDestroy(ev);
+    if (d) (void)hipFree(d);
+    if (h) (void)hipHostFree(h);
+    *this = Upload{};
+  }
+};
+struct Uploads {
+  Upload s[2];
+  int next = 0;
+  ~Uploads() {
+    for (Upload& u : s) u.drop();
+  }
+};
+thread_local Uploads g_uploads;
+
+int upload_slot(size_t bytes, Upload** out) {
+  Upload& u = g_uploads.s[g_uploads.next];
+  g_uploads.next ^= 1;
+  int dev = 0;
+  TQSV_HIP(hipGetDevice(&dev));
+  if (u.cap < bytes || u.dev != dev) {
+    u.drop();
+    const size_t cap = std::max<size_t>(bytes, 64 * 1024);
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&u.h), cap, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&u.d), cap);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&u.ev, hipEventDisableTiming);
+    if (e != hipSuccess) {
+      u.drop();
+      return hip_fail(e, "staging buffers");
+    }
+    u.cap = cap;
+    u.dev = dev;
+  }
+  if (u.busy) {
+    TQSV_HIP(hipEventSynchronize(u.ev));
+    u.busy = false;
+  }
+  *out = &u;
+  return 0;
+}
+
+// marks the slot as read by everything queued on the stream so far
+hipError_t upload_done(Upload* u, hipStream_t st) {
+  hipError_t e = hipEventRecord(u->ev, st);
+  if (e == hipSuccess)
+    u->busy = true;
+  else
+    (void)hipStreamSynchronize(st);
+  return e;
+}
+
+// the staging of a call cannot be part of a captured graph (a replay would
+// read what a later call left there)
+int refuse_capture(hipStream_t st, const char* fn) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  TQSV_HIP(hipStreamIsCapturing(st, &cs));
+  if (cs != hipStreamCaptureStatusNone)
+    return fail(TQSV_EUNSUPPORTED, std::string(fn) + ": not available under stream capture");
   return 0;
 }
 
@@ -144,29 +220,80 @@ int tqsv_apply_kq(const void* psi, void* out, int n, int k, const int* bits, con
     seen |= 1ull << bits[b];
     pos[b] = (uint32_t)bits[b];
   }
+  if ((rc = refuse_capture(S(stream), "tqsv_apply_kq"))) return rc;
+  // Matrix cores for 3 <= k <= 10 with enough other bits for a tile and 16-byte
+  // aligned states; k = 3 runs as k = 4 with the lowest other bit as an
+  // untouched target (U x I: twice the products, but 27 qubits are HBM-bound
+  // either way, 1.47 -> 0.41 ms).  The general kernel keeps what has no such
+  // tile (n below 12, or n - k below 6 for k >= 6: at most 2^15 amplitudes, a
+  // launch's latency) and states at 8-byte alignment.
+  KqGeo geo;
+  std::vector<uint32_t> tb(pos);
+  if (k == 3 && n > 3) {
+    uint32_t b = 0;
+    while ((seen >> b) & 1ull) ++b;
+    tb.push_back(b);
+  }
+  const int kk = (int)tb.size();
+  const bool aligned = ((reinterpret_cast<uintptr_t>(psi) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
+  const bool mfma = aligned && kq_mfma_geo(n, kk, tb.data(), &geo);
   const size_t K = (size_t)1 << k;
-  std::vector<uint64_t> off(K, 0);
-  for (size_t j = 0; j < K; ++j)
-    for (int b = 0; b < k; ++b)
-      if ((j >> (k - 1 - b)) & 1u) off[j] |= 1ull << pos[b];
-  std::vector<float2> u(K * K);
-  for (size_t e = 0; e < K * K; ++e) u[e] = make_float2((float)U[2 * e], (float)U[2 * e + 1]);
-  // per-call device copies of the matrix and tables (freed after the launch completes)
-  const size_t bytes = K * K * sizeof(float2) + K * sizeof(uint64_t) + (size_t)k * sizeof(uint32_t);
-  unsigned char* d = nullptr;
-  TQSV_HIP(hipMalloc(reinterpret_cast<void**>(&d), bytes));
-  float2* dU = reinterpret_cast<float2*>(d);
-  uint64_t* dOff = reinterpret_cast<uint64_t*>(d + K * K * sizeof(float2));
-  uint32_t* dPos = reinterpret_cast<uint32_t*>(d + K * K * sizeof(float2) + K * sizeof(uint64_t));
-  hipError_t e = hipMemcpyAsync(dU, u.data(), K * K * sizeof(float2), hipMemcpyHostToDevice, S(stream));
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(dOff, off.data(), K * sizeof(uint64_t), hipMemcpyHostToDevice, S(stream));
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(dPos, pos.data(), (size_t)k * sizeof(uint32_t), hipMemcpyHostToDevice, S(stream));
-  if (e == hipSuccess) e = k_apply_kq(CF(psi), F(out), n, k, dPos, dOff, dU, S(stream));
-  if (e == hipSuccess) e = hipStreamSynchronize(S(stream));
-  (void)hipFree(d);
+  const size_t KK = (size_t)1 << kk;
+  const size_t bytes = mfma ? KK * KK * sizeof(float2)
+                            : K * K * sizeof(float2) + K * sizeof(uint64_t) + (size_t)k * sizeof(uint32_t);
+  Upload* up = nullptr;
+  if ((rc = upload_slot(bytes, &up))) return rc;
+  float2* hu = reinterpret_cast<float2*>(up->h);
+  if (mfma) {
+    // row/column number by ascending target bits -> index of U (first target
+    // most significant); the added bit of k = 3 gives the block (bit + 1) - 1
+    std::vector<uint32_t> order(kk);
+    for (int b = 0; b < kk; ++b) order[b] = (uint32_t)b;
+    std::sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return tb[x] < tb[y]; });
+    std::vector<uint32_t> ui(KK), extra(KK);
+    for (size_t j = 0; j < KK; ++j) {
+      uint32_t v = 0, e = 0;
+      for (int b = 0; b < kk; ++b)
+        if ((j >> b) & 1u) {
+          if (order[b] < (uint32_t)k)
+            v |= 1u << (k - 1 - order[b]);
+          else
+            e = 1;
+        }
+      ui[j] = v;
+      extra[j] = e;
+    }
+    const size_t chunk = kk < 6 ? KK : 64;
+    float2* o = hu;
+    for (size_t m = 0; m < KK / 16; ++m)
+      for (size_t c = 0; c < KK; c += chunk)
+        for (size_t t = 0; t < chunk; ++t)
+          for (size_t r = 0; r < 16; ++r, ++o) {
+            const size_t row = 16 * m + r, col = c + t;
+            const double* e = U + 2 * ((size_t)ui[row] * K + ui[col]);
+            *o = extra[row] == extra[col] ? make_float2((float)e[0], (float)e[1]) : make_float2(0.f, 0.f);
+          }
+  } else {
+    for (size_t e = 0; e < K * K; ++e) hu[e] = make_float2((float)U[2 * e], (float)U[2 * e + 1]);
+    uint64_t* off = reinterpret_cast<uint64_t*>(hu + K * K);
+    for (size_t j = 0; j < K; ++j) {
+      off[j] = 0;
+      for (int b = 0; b < k; ++b)
+        if ((j >> (k - 1 - b)) & 1u) off[j] |= 1ull << pos[b];
+    }
+    std::memcpy(off + K, pos.data(), (size_t)k * sizeof(uint32_t));
+  }
+  hipError_t e = hipMemcpyAsync(up->d, up->h, bytes, hipMemcpyHostToDevice, S(stream));
+  if (e == hipSuccess) {
+    const float2* dU = reinterpret_cast<const float2*>(up->d);
+    const uint64_t* dOff = reinterpret_cast<const uint64_t*>(dU + K * K);
+    e = mfma ? k_apply_kq_mfma(CF(psi), F(out), kk, geo, dU, S(stream))
+             : k_apply_kq(CF(psi), F(out), n, k, reinterpret_cast<const uint32_t*>(dOff + K), dOff,
+                          dU, S(stream));
+  }
+  const hipError_t er = upload_done(up, S(stream));
   TQSV_HIP(e);
+  TQSV_HIP(er);
   return 0;
 }
 

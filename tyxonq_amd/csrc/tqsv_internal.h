@@ -57,6 +57,24 @@ hipError_t k_scale(float2* psi, int n, float re, float im, hipStream_t st);
 hipError_t k_pad_copy(const float2* src, uint64_t nsrc, float2* dst, uint64_t ndst, hipStream_t st);
 hipError_t k_apply_kq(const float2* psi, float2* out, int n, int k, const uint32_t* bitpos,
                       const uint64_t* off, const float2* U, hipStream_t st);
+// Matrix-core form of the same (tqsv_kq.hip): tiles of 2^KQ_TILE_BITS
+// amplitudes over the lowest targets and the lowest other index bits.
+constexpr int KQ_TILE_BITS = 12;
+struct KqGeo {
+  uint32_t pos[KQ_TILE_BITS];   // index bits of a tile, ascending
+  uint32_t lmap[KQ_TILE_BITS];  // their (linear, swizzled) LDS offsets
+  uint32_t hpos[4];             // targets beyond the 6 lowest (k >= 7)
+  uint32_t skip[16], nskip;     // tile and target bits: a tile number spreads over the others
+  uint32_t nchunk;              // 2^(k-6) chunks of 64 target patterns, at least 1
+  uint32_t ntiles;
+};
+// false: no tile of that shape (few other bits); the general kernel runs
+bool kq_mfma_geo(int n, int k, const uint32_t* bits, KqGeo* geo);
+// A: U's entries per 16-row block m, chunk c and entry pair t: A[(((m *
+// nchunk + c) * NF + t) * 2 + h) * 16 + r] = U[16 m + r][2^LK c + 2 t + h], NF =
+// 2^(LK-1), rows and columns numbered by the target bits in ascending order
+hipError_t k_apply_kq_mfma(const float2* psi, float2* out, int k, const KqGeo& g, const float2* A,
+                           hipStream_t st);
 hipError_t k_probs(const float2* psi, int n, double* out, hipStream_t st);
 // blockwise FP64 partial sums: mode 0 = |psi|^2, 1 = |psi|^2 (-1)^{bit}, 2 = |psi|^2 [bit==keep]
 uint32_t reduce_grid(int n);

@@ -442,7 +442,8 @@ __global__ void ham_apply_kernel(const float2* __restrict__ psi, float2* __restr
 // out[i] = sum_j U[row(i)][j] psi[base(i) | off[j]] for a k-qubit matrix: row
 // is i's target bits (first target most significant), base is i with those
 // bits cleared, off[j] the target bits of column j.  One thread per output
-// amplitude, FP32 sums (out of place).
+// amplitude, FP32 sums (out of place).  For what the matrix-core kernel
+// (tqsv_kq.hip) has no tile for.
 template <typename IDX>
 __global__ void apply_kq_kernel(const float2* __restrict__ psi, float2* __restrict__ out,
                                 uint64_t dim, int k, const uint32_t* __restrict__ bitpos,
