@@ -111,6 +111,27 @@ int tqsv_norm2(const void* psi, int n, double* out, void* stream);
  * Replaces expect_z_statevector, statevector.py:62-68. */
 int tqsv_expect_z(const void* psi, int n, int bit, double* out, void* stream);
 
+/* The same sum written to out_dev[0] (DEVICE) without synchronising;
+ * partials_dev is a device buffer of tqsv_reduce_blocks(n) doubles. */
+int tqsv_reduce_blocks(int n);
+int tqsv_expect_z_dev(const void* psi, int n, int bit, double* partials_dev, double* out_dev,
+                      void* stream);
+
+/* out[i] = 2 ge (-1)^{bit of i} psi[i], ge a double in DEVICE memory: the
+ * gradient of ge * <Z_bit> in psi.  out may be psi. */
+int tqsv_z_grad(const void* psi, void* out, int n, int bit, const double* ge_dev, void* stream);
+
+/* Gate-matrix gradient, k <= 4: G[a][c] = sum over the bits other than `bits`
+ * of g[a] conj(psi[c]), a and c the patterns on `bits` (bits[0] most
+ * significant), 2 * 4^k doubles (re, im) to the host, FP64 products and sums. */
+int tqsv_matrix_grad(const void* psi, const void* g, int n, int k, const int* bits, double* out,
+                     void* stream);
+
+/* tqsv_apply_1q / tqsv_apply_2q out of place (out is a separate state). */
+int tqsv_apply_1q_to(const void* psi, void* out, int n, int bit, const double* U, void* stream);
+int tqsv_apply_2q_to(const void* psi, void* out, int n, int bit_hi, int bit_lo, const double* U,
+                     void* stream);
+
 /* out[0] + i out[1] = sum_i (-1)^{|i & zmask|} conj(u[i]) v[i ^ xmask] (host).
  * With x = z = 0 this is <u|v>; <u|P|v> = (-i)^{|x&z|} times it.  The inner
  * product the reference takes with tensordot(conj(psi'), psi),

@@ -108,6 +108,12 @@ _SIGS = {
     "tqsv_scale": (_I, [_P, _I, _D, _D, _P]),
     "tqsv_norm2": (_I, [_P, _I, _DP, _P]),
     "tqsv_expect_z": (_I, [_P, _I, _I, _DP, _P]),
+    "tqsv_reduce_blocks": (_I, [_I]),
+    "tqsv_expect_z_dev": (_I, [_P, _I, _I, _P, _P, _P]),
+    "tqsv_z_grad": (_I, [_P, _P, _I, _I, _P, _P]),
+    "tqsv_matrix_grad": (_I, [_P, _P, _I, _I, ctypes.POINTER(ctypes.c_int), _DP, _P]),
+    "tqsv_apply_1q_to": (_I, [_P, _P, _I, _I, _DP, _P]),
+    "tqsv_apply_2q_to": (_I, [_P, _P, _I, _I, _I, _DP, _P]),
     "tqsv_dot": (_I, [_P, _P, _I, _U64, _U64, _DP, _P]),
     "tqsv_dot_noalloc": (_I, [_P, _P, _I, _U64, _U64, _P, _P]),
     "tqsv_probs": (_I, [_P, _I, _P, _P]),
@@ -251,6 +257,56 @@ def apply_2q(psi, bit_hi: int, bit_lo: int, U) -> None:
             _ptr(psi), _nqubits(psi), int(bit_hi), int(bit_lo), mat_buffer(U), stream_ptr()
         )
     )
+
+
+def apply_1q_to(psi, bit: int, U):
+    """U psi for a 2x2 matrix as a new state."""
+    out = _torch().empty_like(psi)
+    _check(load().tqsv_apply_1q_to(_ptr(psi), _ptr(out), _nqubits(psi), int(bit), mat_buffer(U),
+                                   stream_ptr()))
+    return out
+
+
+def apply_2q_to(psi, bit_hi: int, bit_lo: int, U):
+    """U psi for a 4x4 matrix as a new state."""
+    out = _torch().empty_like(psi)
+    _check(load().tqsv_apply_2q_to(_ptr(psi), _ptr(out), _nqubits(psi), int(bit_hi), int(bit_lo),
+                                   mat_buffer(U), stream_ptr()))
+    return out
+
+
+def matrix_grad(psi, g, bits: Sequence[int]) -> np.ndarray:
+    """G[a, c] = sum over the other index bits of g[a] conj(psi[c]) (complex128)."""
+    if _nqubits(g) != _nqubits(psi):
+        raise ValueError("state and gradient must have the same length")
+    k = len(bits)
+    out = np.empty((1 << k, 1 << k), dtype=np.complex128)
+    b = (ctypes.c_int * k)(*[int(x) for x in bits])
+    _check(load().tqsv_matrix_grad(_ptr(psi), _ptr(g), _nqubits(psi), k, b,
+                                   out.ctypes.data_as(_DP), stream_ptr()))
+    return out
+
+
+def expect_z_dev(psi, bit: int):
+    """<Z_bit> as a 0-dim float64 tensor on the GPU, without synchronising."""
+    torch = _torch()
+    n = _nqubits(psi)
+    out = torch.empty((), dtype=torch.float64, device=psi.device)
+    part = torch.empty(load().tqsv_reduce_blocks(n), dtype=torch.float64, device=psi.device)
+    _check(load().tqsv_expect_z_dev(_ptr(psi), n, int(bit), part.data_ptr(), out.data_ptr(),
+                                    stream_ptr()))
+    return out
+
+
+def z_grad(psi, bit: int, ge):
+    """2 ge Z_bit psi as a new state; ge a one-element float64 tensor on the GPU."""
+    torch = _torch()
+    if ge.dtype != torch.float64 or not ge.is_cuda or ge.numel() != 1:
+        raise TypeError("expected one float64 on the GPU")
+    out = torch.empty_like(psi)
+    _check(load().tqsv_z_grad(_ptr(psi), _ptr(out), _nqubits(psi), int(bit), ge.data_ptr(),
+                              stream_ptr()))
+    return out
 
 
 def apply_kq(psi, bits: Sequence[int], U):

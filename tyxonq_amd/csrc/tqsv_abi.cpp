@@ -7,6 +7,7 @@
 #include <string>
 #include <vector>
 
+#include "tqsv_grad.h"
 #include "tqsv_planner.h"
 
 namespace tqsv {
@@ -297,6 +298,57 @@ int tqsv_apply_kq(const void* psi, void* out, int n, int k, const int* bits, con
   return 0;
 }
 
+int tqsv_apply_1q_to(const void* psi, void* out, int n, int bit, const double* U, void* stream) {
+  int rc = check_state(psi, n, "tqsv_apply_1q_to");
+  if (rc) return rc;
+  if ((rc = check_bit(bit, n, "tqsv_apply_1q_to"))) return rc;
+  if (!U || !out || out == psi)
+    return fail(TQSV_EINVAL, "tqsv_apply_1q_to: needs a matrix and a separate output state");
+  Mat2f u;
+  for (int j = 0; j < 8; ++j) u.v[j] = (float)U[j];
+  TQSV_HIP(k_apply_1q_to(CF(psi), F(out), n, bit, u, S(stream)));
+  return 0;
+}
+
+int tqsv_apply_2q_to(const void* psi, void* out, int n, int bit_hi, int bit_lo, const double* U,
+                     void* stream) {
+  int rc = check_state(psi, n, "tqsv_apply_2q_to");
+  if (rc) return rc;
+  if ((rc = check_bit(bit_hi, n, "tqsv_apply_2q_to")) || (rc = check_bit(bit_lo, n, "tqsv_apply_2q_to")))
+    return rc;
+  if (bit_hi == bit_lo) return fail(TQSV_EINVAL, "tqsv_apply_2q_to: targets must differ");
+  if (!U || !out || out == psi)
+    return fail(TQSV_EINVAL, "tqsv_apply_2q_to: needs a matrix and a separate output state");
+  Mat4f u;
+  for (int j = 0; j < 32; ++j) u.v[j] = (float)U[j];
+  TQSV_HIP(k_apply_2q_to(CF(psi), F(out), n, bit_hi, bit_lo, u, S(stream)));
+  return 0;
+}
+
+int tqsv_matrix_grad(const void* psi, const void* g, int n, int k, const int* bits, double* out,
+                     void* stream) {
+  int rc = check_state(psi, n, "tqsv_matrix_grad");
+  if (rc) return rc;
+  if ((rc = check_state(g, n, "tqsv_matrix_grad"))) return rc;
+  if (k < 1 || k > 4 || k > n || !bits || !out)
+    return fail(TQSV_EINVAL, "tqsv_matrix_grad: k must be in [1, min(n, 4)]");
+  uint64_t seen = 0;
+  for (int b = 0; b < k; ++b) {
+    if ((rc = check_bit(bits[b], n, "tqsv_matrix_grad"))) return rc;
+    if ((seen >> bits[b]) & 1ull) return fail(TQSV_EINVAL, "tqsv_matrix_grad: repeated target bit");
+    seen |= 1ull << bits[b];
+  }
+  const uint32_t ng = matrix_grad_grid(n, k), nred = 2u << (2 * k);
+  double* d = nullptr;
+  if ((rc = scratch((size_t)(ng + 1) * nred, &d))) return rc;
+  TQSV_HIP(k_matrix_grad(CF(psi), CF(g), n, k, bits, d, S(stream)));
+  TQSV_HIP(k_final_sum(d, ng, nred, d + (size_t)ng * nred, S(stream)));
+  TQSV_HIP(hipMemcpyAsync(out, d + (size_t)ng * nred, nred * sizeof(double), hipMemcpyDeviceToHost,
+                          S(stream)));
+  TQSV_HIP(hipStreamSynchronize(S(stream)));
+  return 0;
+}
+
 int tqsv_apply_diag(void* psi, int n, int nbits, const int* bits, const double* phases,
                     void* stream) {
   int rc = check_state(psi, n, "tqsv_apply_diag");
@@ -364,6 +416,28 @@ int tqsv_expect_z(const void* psi, int n, int bit, double* out, void* stream) {
   if ((rc = check_bit(bit, n, "tqsv_expect_z"))) return rc;
   if (!out) return fail(TQSV_EINVAL, "tqsv_expect_z: out is NULL");
   return reduce_prob_to_host(CF(psi), n, 1, bit, out, S(stream));
+}
+
+int tqsv_reduce_blocks(int n) { return n < 1 || n > 34 ? 0 : (int)reduce_grid(n); }
+
+int tqsv_expect_z_dev(const void* psi, int n, int bit, double* partials_dev, double* out_dev,
+                      void* stream) {
+  int rc = check_state(psi, n, "tqsv_expect_z_dev");
+  if (rc) return rc;
+  if ((rc = check_bit(bit, n, "tqsv_expect_z_dev"))) return rc;
+  if (!partials_dev || !out_dev) return fail(TQSV_EINVAL, "tqsv_expect_z_dev: buffer is NULL");
+  TQSV_HIP(k_reduce_prob(CF(psi), n, 1, bit, partials_dev, S(stream)));
+  TQSV_HIP(k_final_sum(partials_dev, reduce_grid(n), 1, out_dev, S(stream)));
+  return 0;
+}
+
+int tqsv_z_grad(const void* psi, void* out, int n, int bit, const double* ge_dev, void* stream) {
+  int rc = check_state(psi, n, "tqsv_z_grad");
+  if (rc) return rc;
+  if ((rc = check_bit(bit, n, "tqsv_z_grad"))) return rc;
+  if (!out || !ge_dev) return fail(TQSV_EINVAL, "tqsv_z_grad: buffer is NULL");
+  TQSV_HIP(k_z_grad(CF(psi), F(out), n, bit, ge_dev, S(stream)));
+  return 0;
 }
 
 int tqsv_dot(const void* u, const void* v, int n, uint64_t xmask, uint64_t zmask, double* out,

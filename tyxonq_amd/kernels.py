@@ -21,8 +21,7 @@ state or the gate matrix requires grad, the call goes through a
 torch.autograd.Function.  Its backward applies U^dagger to the incoming
 gradient (one more kernel launch) and, for a gate that requires grad, forms
 dL/dU[a, c] = sum_i g[i with target bits a] conj(psi[i with target bits c])
-from 4^k FP64 reductions (tqsv_dot with flip and sign masks on the k target
-bits, then an inverse Walsh-Hadamard transform over the sign masks).
+in one FP64 reduction over both states (tqsv_matrix_grad).
 expect_z_statevector returns a 0-dim float64 tensor on the state's device
 (statevector.py:62-68 returns the backend's scalar), differentiable as well.
 """
@@ -34,7 +33,7 @@ import numpy as np
 
 from . import _native as nat
 
-MAX_GRAD_TARGETS = 4  # 4^k reductions per gate-matrix gradient
+MAX_GRAD_TARGETS = 4  # 4^k sums per gate-matrix gradient
 
 
 def _torch():
@@ -73,40 +72,9 @@ def _apply_new(psi, bits: Sequence[int], U: np.ndarray):
     k = len(bits)
     if k >= 3:
         return nat.apply_kq(psi, list(bits), U)
-    out = psi.clone()
     if k == 1:
-        nat.apply_1q(out, bits[0], U)
-    else:
-        nat.apply_2q(out, bits[0], bits[1], U)
-    return out
-
-
-def _local_mask(v: int, bits: Sequence[int]) -> int:
-    """Global index mask of the local pattern v of U's index (MSB = bits[0])."""
-    k = len(bits)
-    m = 0
-    for j, b in enumerate(bits):
-        if (v >> (k - 1 - j)) & 1:
-            m |= 1 << int(b)
-    return m
-
-
-def _matrix_grad(psi, g, bits: Sequence[int]) -> np.ndarray:
-    """G[a, c] = sum over i with target bits a of g[i] conj(psi[i^a^c]).
-
-    tqsv_dot(psi, g, x, z) = sum_i (-1)^{|i & z|} conj(psi[i]) g[i ^ x]
-    = sum_c (-1)^{c.z} G[c ^ d, c] for the local flip pattern d of x; the
-    inverse Walsh-Hadamard transform over z gives G[c ^ d, c] for every c."""
-    k = len(bits)
-    dim = 1 << k
-    G = np.zeros((dim, dim), dtype=np.complex128)
-    for d in range(dim):
-        xm = _local_mask(d, bits)
-        D = np.array([nat.dot(psi, g, xm, _local_mask(z, bits)) for z in range(dim)])
-        for c in range(dim):
-            sgn = np.array([(-1) ** bin(c & z).count("1") for z in range(dim)], dtype=float)
-            G[c ^ d, c] = np.dot(sgn, D) / dim
-    return G
+        return nat.apply_1q_to(psi, bits[0], U)
+    return nat.apply_2q_to(psi, bits[0], bits[1], U)
 
 
 def _apply_function():
@@ -146,7 +114,7 @@ def _apply_function():
                 gs = gs.reshape(shape)
             if ctx.needs_input_grad[1]:
                 (psi,) = ctx.saved_tensors
-                G = _matrix_grad(psi, g, ctx.bits)
+                G = nat.matrix_grad(psi, g, ctx.bits)
                 dt, dev, shape = ctx.gate_meta
                 gU = torch.as_tensor(G, dtype=torch.complex128).to(device=dev, dtype=dt)
                 gU = gU.reshape(shape)
@@ -164,18 +132,17 @@ def _expect_z_function():
         @staticmethod
         def forward(ctx, state, n, bit):
             psi = _as_state(state, n)
-            val = nat.expect_z(psi, bit)
+            val = nat.expect_z_dev(psi, bit)
             ctx.bit = bit
             ctx.state_meta = (state.dtype, state.device, state.shape)
             ctx.save_for_backward(psi)
-            return torch.tensor(val, dtype=torch.float64, device=state.device)
+            return val.to(state.device)
 
         @staticmethod
         def backward(ctx, ge):
             (psi,) = ctx.saved_tensors
-            zpsi = psi.clone()
-            nat.apply_1q(zpsi, ctx.bit, np.diag([1.0, -1.0]).astype(np.complex128))
-            nat.scale(zpsi, 2.0 * float(ge))
+            g = ge.detach().to(device=psi.device, dtype=torch.float64)
+            zpsi = nat.z_grad(psi, ctx.bit, g)
             dt, dev, shape = ctx.state_meta
             return zpsi.to(device=dev, dtype=dt if dt.is_complex else torch.complex128) \
                 .reshape(shape), None, None
@@ -269,7 +236,7 @@ def expect_z_statevector(state: Any, qubit: int, num_qubits: int, backend: Any =
         return _fn("expz").apply(state, n, bit)
     psi = _as_state(state, n)
     dev = state.device if isinstance(state, torch.Tensor) else psi.device
-    return torch.tensor(nat.expect_z(psi, bit), dtype=torch.float64, device=dev)
+    return nat.expect_z_dev(psi, bit).to(dev)
 
 
 def parameter_shift_gradient(energy_fn: Any, params: Sequence[float]) -> np.ndarray:
