@@ -117,6 +117,17 @@ int tqsv_reduce_blocks(int n);
 int tqsv_expect_z_dev(const void* psi, int n, int bit, double* partials_dev, double* out_dev,
                       void* stream);
 
+/* out[b] = <Z_b> for every index bit b < n (host), in one sweep. */
+int tqsv_expect_z_all(const void* psi, int n, double* out, void* stream);
+
+/* A chain of stochastic one-qubit Kraus channels (kernels/statevector.py:
+ * 132-218), without synchronising: channel c acts on index bit bits[c] with
+ * counts[c] operators (8 doubles each, row-major re/im, all channels
+ * concatenated in `ops`) and keeps the first operator whose cumulative
+ * probability reaches status[c]; the state is normalised. */
+int tqsv_kraus_chain(void* psi, int n, int nchan, const int* bits, const int* counts,
+                     const double* ops, const double* status, void* stream);
+
 /* out[i] = 2 ge (-1)^{bit of i} psi[i], ge a double in DEVICE memory: the
  * gradient of ge * <Z_bit> in psi.  out may be psi. */
 int tqsv_z_grad(const void* psi, void* out, int n, int bit, const double* ge_dev, void* stream);

@@ -110,6 +110,9 @@ _SIGS = {
     "tqsv_expect_z": (_I, [_P, _I, _I, _DP, _P]),
     "tqsv_reduce_blocks": (_I, [_I]),
     "tqsv_expect_z_dev": (_I, [_P, _I, _I, _P, _P, _P]),
+    "tqsv_expect_z_all": (_I, [_P, _I, _DP, _P]),
+    "tqsv_kraus_chain": (_I, [_P, _I, _I, ctypes.POINTER(ctypes.c_int),
+                              ctypes.POINTER(ctypes.c_int), _DP, _DP, _P]),
     "tqsv_z_grad": (_I, [_P, _P, _I, _I, _P, _P]),
     "tqsv_matrix_grad": (_I, [_P, _P, _I, _I, ctypes.POINTER(ctypes.c_int), _DP, _P]),
     "tqsv_apply_1q_to": (_I, [_P, _P, _I, _I, _DP, _P]),
@@ -296,6 +299,31 @@ def expect_z_dev(psi, bit: int):
     _check(load().tqsv_expect_z_dev(_ptr(psi), n, int(bit), part.data_ptr(), out.data_ptr(),
                                     stream_ptr()))
     return out
+
+
+def expect_z_all(psi) -> np.ndarray:
+    """<Z_bit> for every index bit (float64, index = bit)."""
+    n = _nqubits(psi)
+    out = np.empty(n)
+    _check(load().tqsv_expect_z_all(_ptr(psi), n, out.ctypes.data_as(_DP), stream_ptr()))
+    return out
+
+
+def kraus_chain(psi, channels: Sequence[tuple]) -> None:
+    """Stochastic one-qubit channels in order, in place: (bit, 2x2 operators,
+    random number) each.  Queued without synchronising."""
+    c = len(channels)
+    if c == 0:
+        return
+    mats = [np.asarray(K, dtype=np.complex128).reshape(-1)[:4] for _, ks, _ in channels for K in ks]
+    if any(m.size != 4 for m in mats):
+        raise ValueError("Kraus operators must be 2x2")
+    ops = np.ascontiguousarray(np.stack(mats)) if mats else np.zeros((1, 4), dtype=np.complex128)
+    bits = (ctypes.c_int * c)(*[int(b) for b, _, _ in channels])
+    counts = (ctypes.c_int * c)(*[len(ks) for _, ks, _ in channels])
+    st = np.array([float(s) for _, _, s in channels])
+    _check(load().tqsv_kraus_chain(_ptr(psi), _nqubits(psi), c, bits, counts,
+                                   ops.ctypes.data_as(_DP), st.ctypes.data_as(_DP), stream_ptr()))
 
 
 def z_grad(psi, bit: int, ge):

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "tqsv_grad.h"
+#include "tqsv_kraus.h"
 #include "tqsv_planner.h"
 
 namespace tqsv {
@@ -437,6 +438,70 @@ int tqsv_z_grad(const void* psi, void* out, int n, int bit, const double* ge_dev
   if ((rc = check_bit(bit, n, "tqsv_z_grad"))) return rc;
   if (!out || !ge_dev) return fail(TQSV_EINVAL, "tqsv_z_grad: buffer is NULL");
   TQSV_HIP(k_z_grad(CF(psi), F(out), n, bit, ge_dev, S(stream)));
+  return 0;
+}
+
+int tqsv_expect_z_all(const void* psi, int n, double* out, void* stream) {
+  int rc = check_state(psi, n, "tqsv_expect_z_all");
+  if (rc) return rc;
+  if (!out) return fail(TQSV_EINVAL, "tqsv_expect_z_all: out is NULL");
+  const size_t np = zall_doubles(n);
+  double* d = nullptr;
+  if ((rc = scratch(np + (size_t)n, &d))) return rc;
+  TQSV_HIP(k_zall(CF(psi), n, d, d + np, S(stream)));
+  TQSV_HIP(hipMemcpyAsync(out, d + np, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, S(stream)));
+  TQSV_HIP(hipStreamSynchronize(S(stream)));
+  return 0;
+}
+
+int tqsv_kraus_chain(void* psi, int n, int nchan, const int* bits, const int* counts,
+                     const double* ops, const double* status, void* stream) {
+  int rc = check_state(psi, n, "tqsv_kraus_chain");
+  if (rc) return rc;
+  if (nchan < 0 || (nchan > 0 && (!bits || !counts || !ops || !status)))
+    return fail(TQSV_EINVAL, "tqsv_kraus_chain: missing channel data");
+  if (nchan == 0) return 0;
+  size_t nops = 0;
+  for (int c = 0; c < nchan; ++c) {
+    if ((rc = check_bit(bits[c], n, "tqsv_kraus_chain"))) return rc;
+    if (counts[c] < 1) return fail(TQSV_EINVAL, "tqsv_kraus_chain: a channel needs an operator");
+    nops += (size_t)counts[c];
+  }
+  if (nops > (1u << 24)) return fail(TQSV_EINVAL, "tqsv_kraus_chain: too many operators");
+  if ((rc = refuse_capture(S(stream), "tqsv_kraus_chain"))) return rc;
+  // slot: channels, operators, and (device only) the two partial buffers that
+  // the sweeps alternate between
+  const size_t items = (size_t)nchan * sizeof(KrausItem), mats = nops * 8 * sizeof(double);
+  const size_t part = (size_t)kraus_grid(n) * 4;
+  Upload* up = nullptr;
+  if ((rc = upload_slot(items + mats + 2 * part * sizeof(double), &up))) return rc;
+  KrausItem* hi = reinterpret_cast<KrausItem*>(up->h);
+  uint32_t first = 0;
+  for (int c = 0; c < nchan; ++c) {
+    hi[c] = KrausItem{status[c], first, (uint32_t)counts[c]};
+    first += (uint32_t)counts[c];
+  }
+  std::memcpy(up->h + items, ops, mats);
+  const KrausItem* di = reinterpret_cast<const KrausItem*>(up->d);
+  const double* dm = reinterpret_cast<const double*>(up->d + items);
+  double* p0 = reinterpret_cast<double*>(up->d + items + mats);
+  double* p1 = p0 + part;
+  hipError_t e = hipMemcpyAsync(up->d, up->h, items + mats, hipMemcpyHostToDevice, S(stream));
+  bool have = false;  // p0 holds the density matrix of the channel's qubit
+  for (int c = 0; c < nchan && e == hipSuccess; ++c) {
+    if (!have) e = k_kraus_rho(CF(psi), n, bits[c], p0, S(stream));
+    const int next = c + 1 < nchan ? bits[c + 1] : -1;
+    if (e == hipSuccess) e = k_kraus_apply(F(psi), n, bits[c], next, di + c, dm, p0, p1, S(stream));
+    // two channels in a row on one qubit: the pair sweep has formed its
+    // density matrix too
+    have = next >= 0;
+    std::swap(p0, p1);
+  }
+  // the norm of the stored (rounded) result
+  if (e == hipSuccess) e = k_kraus_normalise(F(psi), n, p0, S(stream));
+  const hipError_t er = upload_done(up, S(stream));
+  TQSV_HIP(e);
+  TQSV_HIP(er);
   return 0;
 }
 

@@ -516,38 +516,31 @@ class StatevectorEngine:
         return get_plan(n, ops, tile_bits=self.tile_bits, max_cost=self.max_cost, fuse=self.fuse)
 
     def _execute(self, L: _Lowerer, psi) -> None:
+        chain: List[tuple] = []  # consecutive stochastic channels: one queued chain
         for seg in L.segments:
             kind = seg[0]
+            if kind == "kraus":
+                chain.append(self._channel(seg[1], seg[2], seg[3]))
+                continue
+            nat.kraus_chain(psi, chain)
+            chain = []
             if kind == "ops":
                 self._plan(L.n, seg[1]).run(psi)
             elif kind == "project":
                 nat.project_z(psi, seg[1], seg[2])
-            elif kind == "kraus":
-                self._kraus(psi, seg[1], seg[2], seg[3])
+        nat.kraus_chain(psi, chain)
 
     @staticmethod
-    def _kraus(psi, bit: int, kops: Sequence[np.ndarray], status: Optional[float]) -> None:
-        """Stochastic unravelling (kernels/statevector.py:132-218)."""
-        probs = []
-        for K in kops:
-            tmp = psi.clone()
-            nat.apply_1q(tmp, bit, K)
-            probs.append(nat.norm2(tmp))
-        p = np.asarray(probs, dtype=np.float64)
-        p = p / p.sum()
+    def _channel(bit: int, kops: Sequence[np.ndarray], status: Optional[float]) -> tuple:
+        """One channel of a stochastic unravelling (kernels/statevector.py:132-218)
+        with its random number."""
+        if len(kops) == 0:
+            raise IndexError("a Kraus channel needs at least one operator")
         if status is None:
             import random
 
             status = random.random()
-        sel = 0
-        for i, c in enumerate(np.cumsum(p)):
-            if status <= float(c):
-                sel = i
-                break
-        nat.apply_1q(psi, bit, kops[sel])
-        nrm = nat.norm2(psi)
-        if nrm > 0:
-            nat.scale(psi, 1.0 / math.sqrt(nrm))
+        return bit, kops, float(status)
 
     def _wants_grad(self) -> bool:
         if self.backend.name != "pytorch":
@@ -593,8 +586,11 @@ class StatevectorEngine:
                     "metadata": {"shots": shots, "backend": self.backend.name,
                                  "three_level": bool(kwargs.get("three_level", False))}}
         expectations: Dict[str, float] = {}
+        zs = nat.expect_z_all(psi) if measures else None
         for q in measures:
-            val = nat.expect_z(psi, n - 1 - q)
+            if not 0 <= q < n:
+                raise ValueError(f"measured qubit {q} out of range for n={n}")
+            val = zs[n - 1 - q]
             if z_atten is not None:
                 val *= z_atten[q]
             expectations[f"Z{q}"] = float(val)
