@@ -33,6 +33,12 @@ HIP_FLAGS = [
     "-packed-fp32-ops",
     "-Wno-unused-result",
 ]
+# The interpreting kernels branch on program words only, the same way in every
+# lane: their control flow is left as it is instead of being rewritten into
+# structured form, whose predicate flags and register copies were half of the
+# scalar and a third of the vector instructions of a step.
+INTERP_FLAGS = ["-mllvm", "-structurizecfg-skip-uniform-regions"]
+INTERP_SOURCES = ("tqsv_interp_", "tqsv_batch")
 CXX_FLAGS = [
     "-O2",
     "-std=c++17",
@@ -56,6 +62,10 @@ def sources() -> tuple[list[Path], list[Path]]:
     hip = sorted(CSRC.glob("*.hip"))
     cpp = sorted(CSRC.glob("*.cpp"))
     return hip, cpp
+
+
+def hip_flags(src: Path) -> list[str]:
+    return HIP_FLAGS + (INTERP_FLAGS if src.name.startswith(INTERP_SOURCES) else [])
 
 
 def _stale(src: Path, obj: Path, headers: list[Path]) -> bool:
@@ -98,7 +108,7 @@ def build(verbose: bool = False, incremental: bool = False) -> Path:
     for src in hip:
         obj = OBJ / (src.stem + ".o")
         if not incremental or _stale(src, obj, headers):
-            jobs.append([hipcc, *HIP_FLAGS, "-c", str(src), "-o", str(obj)])
+            jobs.append([hipcc, *hip_flags(src), "-c", str(src), "-o", str(obj)])
     cpp = cpp + [_write_jit_headers()]
     for src in cpp:
         obj = OBJ / (src.stem + ".o")

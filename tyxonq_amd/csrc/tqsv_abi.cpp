@@ -545,13 +545,13 @@ int tqsv_plan_create(int n, const tqsv_op* ops, int nops, const tqsv_plan_opts* 
     p->nu = n;
     p->nops = nops;
     if (opts) {
-      p->so.tile_bits = opts->tile_bits > 0 ? opts->tile_bits : 13;
       p->so.min_low = opts->min_low_bits > 0 ? opts->min_low_bits : 5;
       p->so.max_cost = opts->max_cost > 0 ? opts->max_cost : 0;
       p->so.fuse = opts->fuse != 0;
     }
     p->n = plan_qubits(n, p->so.fuse, opts ? opts->min_qubits : 0);
     p->so.n = p->n;
+    p->so.tile_bits = plan_tile_bits(p->n, opts);
     if (p->n > n) {
       const size_t bytes = sizeof(float2) << p->n;
       TQSV_HIP(hipMalloc(reinterpret_cast<void**>(&p->pad_a), bytes));
@@ -615,13 +615,13 @@ int tqsv_plan_inspect(int n, const tqsv_op* ops, int nops, const tqsv_plan_opts*
     p.nu = n;
     p.nops = nops;
     if (opts) {
-      p.so.tile_bits = opts->tile_bits > 0 ? opts->tile_bits : 13;
       p.so.min_low = opts->min_low_bits > 0 ? opts->min_low_bits : 5;
       p.so.max_cost = opts->max_cost > 0 ? opts->max_cost : 0;
       p.so.fuse = opts->fuse != 0;
     }
     p.n = plan_qubits(n, p.so.fuse, opts ? opts->min_qubits : 0);
     p.so.n = p.n;
+    p.so.tile_bits = plan_tile_bits(p.n, opts);
     std::vector<Gate> g;
     int rc = gates_from_ops(n, ops, nops, g);
     if (rc) return rc;

@@ -192,31 +192,6 @@ __device__ __forceinline__ void u1_apply(float2 (&a)[NSLOT], const M2f& u, const
   }
 }
 
-template <int K, int MODE, typename IDX>
-__device__ __forceinline__ void u1_dispatch(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w,
-                                            const PhaseGeo<IDX>& G) {
-  const uint32_t type = w[2];
-  const bool ctrl = w[3] != 0;
-  const IDX cm = ld_idx<IDX>(w + 4);
-  const IDX cv = ld_idx<IDX>(w + 6);
-  const M2f u = load_m2(w + 8);
-  const bool ton = (G.gb & cm) == (cv & ~G.rmask);
-#define TQSV_U1(TY, CT)                                              \
-  {                                                                 \
-    u1_apply<K, TY, CT, IDX>(a, u, G, cm, cv, ton);                 \
-    if constexpr (MODE == MODE_DUAL) u1_apply<K, TY, CT, IDX>(b, u, G, cm, cv, ton); \
-  }
-  if (ctrl) {
-    if (type == U1_REAL) TQSV_U1(U1_REAL, true)
-    else TQSV_U1(U1_GENERAL, true)
-  } else {
-    if (type == U1_REAL) TQSV_U1(U1_REAL, false)
-    else if (type == U1_RXLIKE) TQSV_U1(U1_RXLIKE, false)
-    else TQSV_U1(U1_GENERAL, false)
-  }
-#undef TQSV_U1
-}
-
 // ---- OP_U2 --------------------------------------------------------------
 template <int KH, int KL, bool CTRL, typename IDX>
 __device__ __forceinline__ void u2_apply(float2 (&a)[NSLOT], cw_t m, const PhaseGeo<IDX>& G,
@@ -248,22 +223,6 @@ __device__ __forceinline__ void u2_apply(float2 (&a)[NSLOT], cw_t m, const Phase
   }
 }
 
-template <int KH, int KL, int MODE, typename IDX>
-__device__ __forceinline__ void u2_dispatch(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w,
-                                            const PhaseGeo<IDX>& G) {
-  const bool ctrl = w[3] != 0;
-  const IDX cm = ld_idx<IDX>(w + 4);
-  const IDX cv = ld_idx<IDX>(w + 6);
-  const bool ton = (G.gb & cm) == (cv & ~G.rmask);
-  if (ctrl) {
-    u2_apply<KH, KL, true, IDX>(a, w + 8, G, cm, cv, ton);
-    if constexpr (MODE == MODE_DUAL) u2_apply<KH, KL, true, IDX>(b, w + 8, G, cm, cv, ton);
-  } else {
-    u2_apply<KH, KL, false, IDX>(a, w + 8, G, cm, cv, ton);
-    if constexpr (MODE == MODE_DUAL) u2_apply<KH, KL, false, IDX>(b, w + 8, G, cm, cv, ton);
-  }
-}
-
 // ---- OP_ROT -------------------------------------------------------------
 template <int K, int MD>
 __device__ __forceinline__ void rot_apply(float2 (&a)[NSLOT], float t) {
@@ -290,30 +249,6 @@ __device__ __forceinline__ void rot_apply(float2 (&a)[NSLOT], float t) {
   }
 }
 
-template <int MODE, typename IDX>
-__device__ __forceinline__ void rot_step(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w,
-                                         const PhaseGeo<IDX>& G) {
-  float t = fl(w + 3);
-  const IDX zs = ld_idx<IDX>(w + 4);
-  if (zs != 0) t = parity((IDX)(G.gb & zs)) ? -t : t;
-#define TQSV_ROT(K, MD)                                  \
-  case 4 * K + MD:                                      \
-    rot_apply<K, MD>(a, t);                             \
-    if constexpr (MODE == MODE_DUAL) rot_apply<K, MD>(b, t); \
-    break;
-#define TQSV_ROTK(K) TQSV_ROT(K, 0) TQSV_ROT(K, 1) TQSV_ROT(K, 2) TQSV_ROT(K, 3)
-  switch (4u * w[1] + w[2]) {
-    TQSV_ROTK(0)
-    TQSV_ROTK(1)
-    TQSV_ROTK(2)
-    TQSV_ROTK(3)
-    TQSV_ROTK(4)
-    default: break;
-  }
-#undef TQSV_ROTK
-#undef TQSV_ROT
-}
-
 // ---- OP_PH --------------------------------------------------------------
 template <int K>
 __device__ __forceinline__ void ph_apply(float2 (&a)[NSLOT], float2 u) {
@@ -327,59 +262,7 @@ __device__ __forceinline__ void ph_apply(float2 (&a)[NSLOT], float2 u) {
 // one loop with a variable slot index, which moves the slot array to scratch.
 #define TQSV_ARM_END(TAG, K) __asm__ volatile("; " TAG " arm %0" ::"n"(K))
 
-// Marks every slot register as rewritten in place.  Used at the end of switch
-// arms that leave some slots untouched, so that all arms hand the slots over
-// in the same registers instead of each needing copies at the join.
-__device__ __forceinline__ void touch_all(float2 (&a)[NSLOT]) {
-#pragma unroll
-  for (int s = 0; s < NSLOT; ++s) __asm__ volatile("" : "+v"(a[s].x), "+v"(a[s].y));
-}
-
-template <int MODE, typename IDX>
-__device__ __forceinline__ void ph_step(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w,
-                                        const PhaseGeo<IDX>& G) {
-  float2 u = make_float2(fl(w + 4), fl(w + 5));
-  const uint32_t nent = w[2];
-  cw_t e = w + OPH_HDR;
-  for (uint32_t i = 0; i < nent; ++i, e += OPH_ENT) {
-    const float2 v = cmul(u, make_float2(fl(e + 1), fl(e + 2)));
-    const bool on = ((G.gb >> e[0]) & 1u) != 0;
-    u = sel2(on, v, u);
-  }
-#define TQSV_PH(K)                                       \
-  case K:                                               \
-    ph_apply<K>(a, u);                                  \
-    touch_all(a);                                       \
-    if constexpr (MODE == MODE_DUAL) {                  \
-      ph_apply<K>(b, u);                                \
-      touch_all(b);                                     \
-    }                                                   \
-    TQSV_ARM_END("ph", K);                              \
-    break;
-  switch (w[1]) {
-    TQSV_PH(0)
-    TQSV_PH(1)
-    TQSV_PH(2)
-    TQSV_PH(3)
-    TQSV_PH(4)
-    default: break;
-  }
-#undef TQSV_PH
-}
-
 // ---- OP_SGN / OP_TAB / OP_THR ---------------------------------------------
-template <int MODE>
-__device__ __forceinline__ void sgn_step(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w) {
-  const uint32_t mask = w[1];
-#pragma unroll
-  for (int s = 0; s < NSLOT; ++s) {
-    if (mask & (1u << s)) {
-      a[s] = cneg(a[s]);
-      if constexpr (MODE == MODE_DUAL) b[s] = cneg(b[s]);
-    }
-  }
-}
-
 template <int MODE>
 __device__ __forceinline__ void tab_step(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w) {
   cw_t t = w + TAB_OFF;
@@ -388,24 +271,6 @@ __device__ __forceinline__ void tab_step(float2 (&a)[NSLOT], float2 (&b)[NSLOT],
     const float2 f = make_float2(fl(t + 2 * s), fl(t + 2 * s + 1));
     a[s] = cmul(a[s], f);
     if constexpr (MODE == MODE_DUAL) b[s] = cmul(b[s], f);
-  }
-}
-
-template <int MODE, typename IDX>
-__device__ __forceinline__ void thr_step(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w,
-                                         const PhaseGeo<IDX>& G) {
-  const uint32_t nent = w[1];
-  float2 F = make_float2(fl(w + 2), fl(w + 3));
-  cw_t e = w + THR_HDR;
-  for (uint32_t i = 0; i < nent; ++i, e += THR_ENT) {
-    const float2 v = cmul(F, make_float2(fl(e + 2), fl(e + 3)));
-    const bool on = (((G.gb >> e[0]) & (G.gb >> e[1])) & 1u) != 0;
-    F = sel2(on, v, F);
-  }
-#pragma unroll
-  for (int s = 0; s < NSLOT; ++s) {
-    a[s] = cmul(a[s], F);
-    if constexpr (MODE == MODE_DUAL) b[s] = cmul(b[s], F);
   }
 }
 
@@ -448,59 +313,6 @@ __device__ __forceinline__ bool cxp_thread_on(cw_t w, const PhaseGeo<IDX>& G) {
   const IDX cm = ld_idx<IDX>(w + 4);
   const IDX cv = ld_idx<IDX>(w + 6);
   return (G.gb & cm) == cv;
-}
-
-// interpreter form: smask (bit s: the register part of the control holds
-// for slot s) is uniform, ton is the thread part.  Dual passes swap both
-// states per pair, so that each pair's selector dies at once.  (Arms per
-// control slot would not be cheaper here: every arm must hand the slots over
-// in the same registers, so a renaming turns into moves at the join.)
-template <int K, bool DUAL>
-__device__ __forceinline__ void cxp_apply_rt(float2 (&a)[NSLOT], float2 (&b)[NSLOT], bool ton,
-                                             uint32_t smask) {
-#pragma unroll
-  for (int s = 0; s < NSLOT; ++s) {
-    if (s & (1 << K)) continue;
-    const int s1 = s | (1 << K);
-    const bool on = ((smask >> s) & 1u) != 0 && ton;
-    const float2 x0 = a[s], x1 = a[s1];
-    a[s] = sel2(on, x1, x0);
-    a[s1] = sel2(on, x0, x1);
-    if constexpr (DUAL) {
-      const float2 y0 = b[s], y1 = b[s1];
-      b[s] = sel2(on, y1, y0);
-      b[s1] = sel2(on, y0, y1);
-    }
-  }
-}
-
-template <int K, int MODE, typename IDX>
-__device__ __forceinline__ void cxp_dispatch(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w,
-                                             const PhaseGeo<IDX>& G) {
-  const uint32_t smask = w[8];
-  const bool ton = w[2] == CX_THREAD ? cxp_thread_on<IDX>(w, G) : true;
-  cxp_apply_rt<K, MODE == MODE_DUAL>(a, b, ton, smask);
-}
-
-template <int MODE, typename IDX>
-__device__ __forceinline__ void cxp_switch(uint32_t k, float2 (&a)[NSLOT], float2 (&b)[NSLOT],
-                                           cw_t w, const PhaseGeo<IDX>& G) {
-#define TQSV_CXP(K)                                \
-  case K:                                          \
-    cxp_dispatch<K, MODE, IDX>(a, b, w, G);        \
-    touch_all(a);                                  \
-    if constexpr (MODE == MODE_DUAL) touch_all(b); \
-    TQSV_ARM_END("cxp", K);                        \
-    break;
-  switch (k) {
-    TQSV_CXP(0)
-    TQSV_CXP(1)
-    TQSV_CXP(2)
-    TQSV_CXP(3)
-    TQSV_CXP(4)
-    default: break;
-  }
-#undef TQSV_CXP
 }
 
 // generated-kernel form: slot, control slot and value fixed at compile time
@@ -573,38 +385,6 @@ __device__ __forceinline__ void prot_apply1(float2 (&a)[NSLOT], const PhaseGeo<I
   }
 }
 
-template <int XR, int MODE, typename IDX>
-__device__ __forceinline__ void prot_x(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w,
-                                       const PhaseGeo<IDX>& G) {
-  const IDX z = ld_idx<IDX>(w + 2);
-  const float c = fl(w + 4), sn = fl(w + 5);
-  const uint32_t k = w[6] & 3u;
-  const uint32_t q = (k + 3u) & 3u;  // -i * i^k
-  const uint32_t xzpar = k & 1u;
-#define TQSV_PR(QQ)                                          \
-  {                                                         \
-    prot_apply1<XR, QQ, IDX>(a, G, z, c, sn, xzpar);         \
-    if constexpr (MODE == MODE_DUAL) prot_apply1<XR, QQ, IDX>(b, G, z, c, sn, xzpar); \
-  }
-  if constexpr (XR == 0) {
-    TQSV_PR(3)
-  } else {
-    // i^(q+2) = -i^q: the sign goes into s, so two arms per flip mask suffice
-    const float snq = q >= 2u ? -sn : sn;
-#define TQSV_PRS(QQ)                                           \
-  {                                                           \
-    prot_apply1<XR, QQ, IDX>(a, G, z, c, snq, xzpar);          \
-    if constexpr (MODE == MODE_DUAL) prot_apply1<XR, QQ, IDX>(b, G, z, c, snq, xzpar); \
-  }
-    if (q & 1u)
-      TQSV_PRS(1)
-    else
-      TQSV_PRS(0)
-#undef TQSV_PRS
-  }
-#undef TQSV_PR
-}
-
 // ---- OP_PGRP ------------------------------------------------------------
 // compressed index of slot s over the slot bits of mask M (ascending)
 template <uint32_t M>
@@ -623,13 +403,12 @@ __device__ __forceinline__ constexpr uint32_t pext_slot(uint32_t s) {
 // new_j = a_j + (cm1 a_j + sg(i) u_i a_i), the small bracket first so that
 // each amplitude is rounded once at its own size.  sg(i) = (-1)^{tp + bit s of
 // the slot sign mask}, tp the parity of the thread's bits & z0.
-// CT (generated kernels): the active class mask ACT, the slot sign mask SM
-// and |x & z0| mod 2 KP are compile-time constants, so the slot signs become
-// FMA source modifiers and only tp is applied at run time (once per class).
-// Otherwise they are the uniform runtime values act, sm, kpar.
-template <int XR, bool CT, uint32_t ACT, uint32_t SM, uint32_t KP, typename IDX>
+// The active class mask ACT, the slot sign mask SM and |x & z0| mod 2 KP are
+// compile-time constants, so the slot signs become FMA source modifiers and
+// only tp is applied at run time (once per class).
+template <int XR, uint32_t ACT, uint32_t SM, uint32_t KP, typename IDX>
 __device__ __forceinline__ void pgrp_apply1(float2 (&a)[NSLOT], const PhaseGeo<IDX>& G, IDX z0,
-                                            uint32_t kpar, uint32_t act, uint32_t sm, cw_t tab) {
+                                            cw_t tab) {
   constexpr int LB = XR & (-XR);
   constexpr uint32_t HI = (uint32_t)XR & ~(uint32_t)LB;
   const uint32_t tp = parity((IDX)(G.gb & z0));
@@ -637,29 +416,17 @@ __device__ __forceinline__ void pgrp_apply1(float2 (&a)[NSLOT], const PhaseGeo<I
   for (int s = 0; s < NSLOT; ++s) {
     if (s & LB) continue;
     const uint32_t cls = pext_slot<HI>((uint32_t)s);
-    if (CT ? !((ACT >> cls) & 1u) : !((act >> cls) & 1u)) continue;
+    if (!((ACT >> cls) & 1u)) continue;
     const int s1 = s ^ XR;
     const cw_t e = tab + PG_ENT * cls;
     const float cm1 = fl(e);
-    float uir, uii, ujr, uji;
-    if constexpr (CT) {
-      // the thread sign once per class (common subexpression across the
-      // class's pairs), the slot signs at compile time
-      const float tir = tp ? -fl(e + 1) : fl(e + 1), tii = tp ? -fl(e + 2) : fl(e + 2);
-      const float tjr = tp ? -fl(e + 3) : fl(e + 3), tji = tp ? -fl(e + 4) : fl(e + 4);
-      const bool bi = (SM >> s) & 1u, bj = bi != ((KP & 1u) != 0u);
-      uir = bi ? -tir : tir;
-      uii = bi ? -tii : tii;
-      ujr = bj ? -tjr : tjr;
-      uji = bj ? -tji : tji;
-    } else {
-      const uint32_t sgi = tp ^ ((sm >> s) & 1u);
-      const uint32_t sgj = sgi ^ kpar;
-      uir = sgi ? -fl(e + 1) : fl(e + 1);
-      uii = sgi ? -fl(e + 2) : fl(e + 2);
-      ujr = sgj ? -fl(e + 3) : fl(e + 3);
-      uji = sgj ? -fl(e + 4) : fl(e + 4);
-    }
+    // the thread sign once per class (common subexpression across the
+    // class's pairs), the slot signs at compile time
+    const float tir = tp ? -fl(e + 1) : fl(e + 1), tii = tp ? -fl(e + 2) : fl(e + 2);
+    const float tjr = tp ? -fl(e + 3) : fl(e + 3), tji = tp ? -fl(e + 4) : fl(e + 4);
+    const bool bi = (SM >> s) & 1u, bj = bi != ((KP & 1u) != 0u);
+    const float uir = bi ? -tir : tir, uii = bi ? -tii : tii;
+    const float ujr = bj ? -tjr : tjr, uji = bj ? -tji : tji;
     const float2 x0 = a[s], x1 = a[s1];
     const float t0r = fmaf(-uji, x1.y, fmaf(cm1, x0.x, ujr * x1.x));
     const float t0i = fmaf(uji, x1.x, fmaf(cm1, x0.y, ujr * x1.y));
@@ -670,68 +437,35 @@ __device__ __forceinline__ void pgrp_apply1(float2 (&a)[NSLOT], const PhaseGeo<I
   }
 }
 
-template <int XR, int MODE, typename IDX>
-__device__ __forceinline__ void pgrp_x(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w,
-                                       const PhaseGeo<IDX>& G) {
-  if constexpr (XR != 0) {
-    const IDX z0 = ld_idx<IDX>(w + 2);
-    const uint32_t kpar = w[4], act = w[5], sm = w[6];
-    pgrp_apply1<XR, false, 0u, 0u, 0u, IDX>(a, G, z0, kpar, act, sm, w + PG_HDR);
-    if constexpr (MODE == MODE_DUAL)
-      pgrp_apply1<XR, false, 0u, 0u, 0u, IDX>(b, G, z0, kpar, act, sm, w + PG_HDR);
-  }
-}
-
 // ---- OP_RED -------------------------------------------------------------
 // +-1.0 from bit s of a uniform mask, built with scalar bit operations
 __device__ __forceinline__ float sgn1(uint32_t mask, int s) {
   return __uint_as_float(0x3f800000u | (((mask >> s) & 1u) << 31));
 }
 
-// Per term: FP32 sum over the thread's 32 slots, then FP64 over the wave's
-// lanes, the LDS accumulator of the wave and beyond.
-// Cross reduction of a dual pass (one entry): one part (PART 0 real, 1
+// Cross reduction of a dual pass in a generated kernel: one part (PART 0 real, 1
 // imaginary) of sum_s sg(s) conj(b[s]) a[s ^ XR], the part the gradient of
-// the rotation needs.  Two FP32 accumulators (even and odd slots) keep the
-// FMA chains short.  CT: the slot sign mask SM is a compile-time constant
-// (generated kernels; the signs become FMA source modifiers), else the
-// uniform runtime mask `sm`.
-template <int XR, int PART, bool CT, uint32_t SM>
-__device__ __forceinline__ float cross_part(const float2 (&a)[NSLOT], const float2 (&b)[NSLOT],
-                                            uint32_t sm) {
+// the rotation needs, in FP32 over the thread's 32 slots, then FP64 over the
+// wave's lanes, the LDS accumulator of the wave and beyond.  Two FP32
+// accumulators (even and odd slots) keep the FMA chains short; the slot sign
+// mask SM becomes FMA source modifiers.
+template <int XR, int PART, uint32_t SM>
+__device__ __forceinline__ float cross_part(const float2 (&a)[NSLOT], const float2 (&b)[NSLOT]) {
   float v[2] = {0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < NSLOT; ++s) {
     const float2 u = b[s], w = a[s ^ XR];  // conj(u) * w
     float& acc = v[s & 1];
-    if constexpr (CT) {
-      const bool neg = (SM >> s) & 1u;
-      if constexpr (PART == 0) {
-        acc = fmaf(neg ? -u.x : u.x, w.x, acc);
-        acc = fmaf(neg ? -u.y : u.y, w.y, acc);
-      } else {
-        acc = fmaf(neg ? -u.x : u.x, w.y, acc);
-        acc = fmaf(neg ? u.y : -u.y, w.x, acc);
-      }
+    const bool neg = (SM >> s) & 1u;
+    if constexpr (PART == 0) {
+      acc = fmaf(neg ? -u.x : u.x, w.x, acc);
+      acc = fmaf(neg ? -u.y : u.y, w.y, acc);
     } else {
-      const float q = PART == 0 ? u.x * w.x + u.y * w.y : u.x * w.y - u.y * w.x;
-      acc = fmaf(sgn1(sm, s), q, acc);
+      acc = fmaf(neg ? -u.x : u.x, w.y, acc);
+      acc = fmaf(neg ? u.y : -u.y, w.x, acc);
     }
   }
   return v[0] + v[1];
-}
-
-template <int XR, typename IDX>
-__device__ __forceinline__ void red_cross(const float2 (&a)[NSLOT], const float2 (&b)[NSLOT],
-                                          cw_t w, const PhaseGeo<IDX>& G, double* acc,
-                                          uint32_t nred) {
-  cw_t e = w + RED_HDR;
-  const IDX zt = ld_idx<IDX>(e + 1);
-  float v = e[4] ? cross_part<XR, 1, false, 0u>(a, b, e[3]) : cross_part<XR, 0, false, 0u>(a, b, e[3]);
-  if (parity((IDX)(G.gb & zt))) v = -v;
-  const double d = wave_sum_last_d((double)v);
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  if (lane == 63) acc[wave * nred + e[0]] += d;
 }
 
 // the cross reduction of generated kernels: slot, z mask, sign mask and part
@@ -739,16 +473,66 @@ __device__ __forceinline__ void red_cross(const float2 (&a)[NSLOT], const float2
 template <int XR, int PART, uint32_t SM, uint32_t SLOT, uint32_t NRED, typename IDX>
 __device__ __forceinline__ void jred_cross(const float2 (&a)[NSLOT], const float2 (&b)[NSLOT],
                                            const PhaseGeo<IDX>& G, IDX zt, double* acc) {
-  float v = cross_part<XR, PART, true, SM>(a, b, 0u);
+  float v = cross_part<XR, PART, SM>(a, b);
   if (parity((IDX)(G.gb & zt))) v = -v;
   const double d = wave_sum_last_d((double)v);
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   if (lane == 63) acc[wave * NRED + SLOT] += d;
 }
 
-template <int XR, int KIND, int MODE, typename IDX>
-__device__ __forceinline__ void red_x(const float2 (&a)[NSLOT], const float2 (&b)[NSLOT], cw_t w,
-                                      const PhaseGeo<IDX>& G, double* acc, uint32_t nred) {
+// Group reduction of a dual pass (kind RED_GROUP): Im <lambda| G |psi> for
+// the generator G = sum_r g_r P_r of a rotation group with one shared
+// parameter, in one sweep over the thread's pairs and one wave sum, instead
+// of one reduction (two wave sums) per Pauli string.  ACT, SM and KP as for pgrp_apply1.
+template <int XR, uint32_t ACT, uint32_t SM, uint32_t KP, typename IDX>
+__device__ __forceinline__ float group_part(const float2 (&a)[NSLOT], const float2 (&b)[NSLOT],
+                                            const PhaseGeo<IDX>& G, IDX z0, cw_t tab) {
+  constexpr int LB = XR & (-XR);
+  constexpr uint32_t HI = (uint32_t)XR & ~(uint32_t)LB;
+  const uint32_t tp = parity((IDX)(G.gb & z0));
+  float vi = 0.f;
+#pragma unroll
+  for (int s = 0; s < NSLOT; ++s) {
+    if (s & LB) continue;
+    const uint32_t cls = pext_slot<HI>((uint32_t)s);
+    if (!((ACT >> cls) & 1u)) continue;
+    const int s1 = s ^ XR;
+    cw_t c = tab + RGRP_ENT * cls;
+    const float tir = tp ? -fl(c) : fl(c), tii = tp ? -fl(c + 1) : fl(c + 1);
+    const float tjr = tp ? -fl(c + 2) : fl(c + 2), tji = tp ? -fl(c + 3) : fl(c + 3);
+    const bool bi = (SM >> s) & 1u, bj = bi != ((KP & 1u) != 0u);
+    const float wir = bi ? -tir : tir, wii = bi ? -tii : tii;
+    const float wjr = bj ? -tjr : tjr, wji = bj ? -tji : tji;
+    // Im(conj(l) w a) = l.x (w.r a.y + w.i a.x) - l.y (w.r a.x - w.i a.y)
+    const float2 li = b[s], lj = b[s1], ai = a[s], aj = a[s1];
+    const float qjr = wjr * aj.x - wji * aj.y, qji = wjr * aj.y + wji * aj.x;
+    const float qir = wir * ai.x - wii * ai.y, qii = wir * ai.y + wii * ai.x;
+    vi = fmaf(li.x, qji, vi);
+    vi = fmaf(-li.y, qjr, vi);
+    vi = fmaf(lj.x, qii, vi);
+    vi = fmaf(-lj.y, qir, vi);
+  }
+  return vi;
+}
+
+// the group reduction of generated kernels
+template <int XR, uint32_t ACT, uint32_t SM, uint32_t KP, uint32_t SLOT, uint32_t NRED,
+          typename IDX>
+__device__ __forceinline__ void jred_group(const float2 (&a)[NSLOT], const float2 (&b)[NSLOT],
+                                           cw_t w, const PhaseGeo<IDX>& G, IDX z0, double* acc) {
+  const float vi =
+      group_part<XR, ACT, SM, KP, IDX>(a, b, G, z0, w + RED_HDR + RED_ENT + 2);
+  const double d = wave_sum_last_d((double)vi);
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  if (lane == 63) acc[wave * NRED + SLOT] += d;
+}
+
+// Per term of an expectation pass: FP32 sum over the thread's slots (pairs for
+// KIND = RED_PAIR), then FP64 over the wave's lanes, the LDS accumulator of the
+// wave and beyond.
+template <int XR, int KIND, typename IDX>
+__device__ __forceinline__ void red_x(const float2 (&a)[NSLOT], cw_t w, const PhaseGeo<IDX>& G,
+                                      double* acc, uint32_t nred) {
   constexpr int LB = XR & (-XR);
   float2 p[NSLOT];
 #pragma unroll
@@ -757,13 +541,8 @@ __device__ __forceinline__ void red_x(const float2 (&a)[NSLOT], const float2 (&b
       if (s & LB) continue;
       const float2 u = a[s ^ XR], v = a[s];  // conj(u) * v
       p[s] = make_float2(u.x * v.x + u.y * v.y, u.x * v.y - u.y * v.x);
-    } else if constexpr (KIND == RED_DIAG) {
-      p[s] = make_float2(a[s].x * a[s].x + a[s].y * a[s].y, 0.f);
     } else {
-      if constexpr (MODE == MODE_DUAL) {
-        const float2 u = b[s], v = a[s ^ XR];
-        p[s] = make_float2(u.x * v.x + u.y * v.y, u.x * v.y - u.y * v.x);
-      }
+      p[s] = make_float2(a[s].x * a[s].x + a[s].y * a[s].y, 0.f);
     }
   }
   const uint32_t nterms = w[3];
@@ -794,167 +573,19 @@ __device__ __forceinline__ void red_x(const float2 (&a)[NSLOT], const float2 (&b
   }
 }
 
-// Group reduction of a dual pass (kind RED_GROUP): Im <lambda| G |psi> for
-// the generator G = sum_r g_r P_r of a rotation group with one shared
-// parameter, in one sweep over the thread's pairs and one wave sum, instead
-// of one reduction (two wave sums) per Pauli string.  CT: active class mask,
-// slot sign mask and kpar fixed at compile time (as for pgrp_apply1).
-template <int XR, bool CT, uint32_t ACT, uint32_t SM, uint32_t KP, typename IDX>
-__device__ __forceinline__ float group_part(const float2 (&a)[NSLOT], const float2 (&b)[NSLOT],
-                                            const PhaseGeo<IDX>& G, IDX z0, uint32_t kpar,
-                                            uint32_t act, uint32_t sm, cw_t tab) {
-  constexpr int LB = XR & (-XR);
-  constexpr uint32_t HI = (uint32_t)XR & ~(uint32_t)LB;
-  const uint32_t tp = parity((IDX)(G.gb & z0));
-  float vi = 0.f;
-#pragma unroll
-  for (int s = 0; s < NSLOT; ++s) {
-    if (s & LB) continue;
-    const uint32_t cls = pext_slot<HI>((uint32_t)s);
-    if (CT ? !((ACT >> cls) & 1u) : !((act >> cls) & 1u)) continue;
-    const int s1 = s ^ XR;
-    cw_t c = tab + RGRP_ENT * cls;
-    float wir, wii, wjr, wji;
-    if constexpr (CT) {
-      const float tir = tp ? -fl(c) : fl(c), tii = tp ? -fl(c + 1) : fl(c + 1);
-      const float tjr = tp ? -fl(c + 2) : fl(c + 2), tji = tp ? -fl(c + 3) : fl(c + 3);
-      const bool bi = (SM >> s) & 1u, bj = bi != ((KP & 1u) != 0u);
-      wir = bi ? -tir : tir;
-      wii = bi ? -tii : tii;
-      wjr = bj ? -tjr : tjr;
-      wji = bj ? -tji : tji;
-    } else {
-      const uint32_t sgi = tp ^ ((sm >> s) & 1u);
-      const uint32_t sgj = sgi ^ kpar;
-      wjr = sgj ? -fl(c + 2) : fl(c + 2);
-      wji = sgj ? -fl(c + 3) : fl(c + 3);
-      wir = sgi ? -fl(c) : fl(c);
-      wii = sgi ? -fl(c + 1) : fl(c + 1);
-    }
-    // Im(conj(l) w a) = l.x (w.r a.y + w.i a.x) - l.y (w.r a.x - w.i a.y)
-    const float2 li = b[s], lj = b[s1], ai = a[s], aj = a[s1];
-    const float qjr = wjr * aj.x - wji * aj.y, qji = wjr * aj.y + wji * aj.x;
-    const float qir = wir * ai.x - wii * ai.y, qii = wir * ai.y + wii * ai.x;
-    vi = fmaf(li.x, qji, vi);
-    vi = fmaf(-li.y, qjr, vi);
-    vi = fmaf(lj.x, qii, vi);
-    vi = fmaf(-lj.y, qir, vi);
-  }
-  return vi;
-}
-
-template <int XR, typename IDX>
-__device__ __forceinline__ void red_group(const float2 (&a)[NSLOT], const float2 (&b)[NSLOT],
-                                          cw_t w, const PhaseGeo<IDX>& G, double* acc,
-                                          uint32_t nred) {
-  cw_t e = w + RED_HDR;
-  cw_t t = e + RED_ENT;
-  const float vi = group_part<XR, false, 0u, 0u, 0u, IDX>(a, b, G, ld_idx<IDX>(e + 1), t[0], t[1],
-                                                          e[3], t + 2);
-  const double d = wave_sum_last_d((double)vi);
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  if (lane == 63) acc[wave * nred + e[0]] += d;
-}
-
-// the group reduction of generated kernels
-template <int XR, uint32_t ACT, uint32_t SM, uint32_t KP, uint32_t SLOT, uint32_t NRED,
-          typename IDX>
-__device__ __forceinline__ void jred_group(const float2 (&a)[NSLOT], const float2 (&b)[NSLOT],
-                                           cw_t w, const PhaseGeo<IDX>& G, IDX z0, double* acc) {
-  const float vi =
-      group_part<XR, true, ACT, SM, KP, IDX>(a, b, G, z0, 0u, 0u, 0u, w + RED_HDR + RED_ENT + 2);
-  const double d = wave_sum_last_d((double)vi);
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  if (lane == 63) acc[wave * NRED + SLOT] += d;
-}
-
-template <int XR, int MODE, typename IDX>
-__device__ __forceinline__ void red_dispatch_kind(const float2 (&a)[NSLOT],
-                                                  const float2 (&b)[NSLOT], cw_t w,
-                                                  const PhaseGeo<IDX>& G, double* acc,
-                                                  uint32_t nred) {
-  const uint32_t kind = w[2];
-  if constexpr (MODE == MODE_DUAL) {
-    if (kind == RED_CROSS) red_cross<XR, IDX>(a, b, w, G, acc, nred);
-    if constexpr (XR != 0)
-      if (kind == RED_GROUP) red_group<XR, IDX>(a, b, w, G, acc, nred);
-  } else {
-    if constexpr (XR == 0) {
-      red_x<0, RED_DIAG, MODE, IDX>(a, b, w, G, acc, nred);
-    } else {
-      red_x<XR, RED_PAIR, MODE, IDX>(a, b, w, G, acc, nred);
-    }
-  }
-}
-
-// ---- dispatch helpers over the runtime register masks --------------------
-template <int MODE, typename IDX, int X = 0>
-__device__ __forceinline__ void prot_switch(uint32_t xr, float2 (&a)[NSLOT], float2 (&b)[NSLOT],
-                                            cw_t w, const PhaseGeo<IDX>& G) {
-  if constexpr (X < NSLOT) {
-    if (xr == (uint32_t)X) {
-      prot_x<X, MODE, IDX>(a, b, w, G);
-      return;
-    }
-    prot_switch<MODE, IDX, X + 1>(xr, a, b, w, G);
-  }
-}
-
-template <int MODE, typename IDX, int X = 0>
-__device__ __forceinline__ void pgrp_switch(uint32_t xr, float2 (&a)[NSLOT], float2 (&b)[NSLOT],
-                                            cw_t w, const PhaseGeo<IDX>& G) {
-  if constexpr (X < NSLOT) {
-    if (xr == (uint32_t)X) {
-      pgrp_x<X, MODE, IDX>(a, b, w, G);
-      __asm__ volatile("; pgrp arm %0" ::"n"(X));
-      return;
-    }
-    pgrp_switch<MODE, IDX, X + 1>(xr, a, b, w, G);
-  }
-}
-
-template <int MODE, typename IDX, int X = 0>
-__device__ __forceinline__ void red_switch(uint32_t xr, const float2 (&a)[NSLOT],
-                                           const float2 (&b)[NSLOT], cw_t w,
+// dispatch over the runtime register mask
+template <typename IDX, int X = 0>
+__device__ __forceinline__ void red_switch(uint32_t xr, const float2 (&a)[NSLOT], cw_t w,
                                            const PhaseGeo<IDX>& G, double* acc, uint32_t nred) {
   if constexpr (X < NSLOT) {
     if (xr == (uint32_t)X) {
-      red_dispatch_kind<X, MODE, IDX>(a, b, w, G, acc, nred);
+      red_x<X, X == 0 ? (int)RED_DIAG : (int)RED_PAIR, IDX>(a, w, G, acc, nred);
       // keeps the arms distinct: merged arms index the slot array with a
       // variable, which moves it to scratch memory
       __asm__ volatile("; red arm %0" ::"n"(X));
       return;
     }
-    red_switch<MODE, IDX, X + 1>(xr, a, b, w, G, acc, nred);
-  }
-}
-
-template <int MODE, typename IDX>
-__device__ __forceinline__ void u1_switch(uint32_t k, float2 (&a)[NSLOT], float2 (&b)[NSLOT],
-                                          cw_t w, const PhaseGeo<IDX>& G) {
-  switch (k) {
-    case 0: u1_dispatch<0, MODE, IDX>(a, b, w, G); break;
-    case 1: u1_dispatch<1, MODE, IDX>(a, b, w, G); break;
-    case 2: u1_dispatch<2, MODE, IDX>(a, b, w, G); break;
-    case 3: u1_dispatch<3, MODE, IDX>(a, b, w, G); break;
-    default: u1_dispatch<4, MODE, IDX>(a, b, w, G); break;
-  }
-}
-
-template <int MODE, typename IDX>
-__device__ __forceinline__ void u2_switch(uint32_t kh, uint32_t kl, float2 (&a)[NSLOT],
-                                          float2 (&b)[NSLOT], cw_t w, const PhaseGeo<IDX>& G) {
-  switch (kh * 8u + kl) {
-    case 8 * 1 + 0: u2_dispatch<1, 0, MODE, IDX>(a, b, w, G); break;
-    case 8 * 2 + 0: u2_dispatch<2, 0, MODE, IDX>(a, b, w, G); break;
-    case 8 * 2 + 1: u2_dispatch<2, 1, MODE, IDX>(a, b, w, G); break;
-    case 8 * 3 + 0: u2_dispatch<3, 0, MODE, IDX>(a, b, w, G); break;
-    case 8 * 3 + 1: u2_dispatch<3, 1, MODE, IDX>(a, b, w, G); break;
-    case 8 * 3 + 2: u2_dispatch<3, 2, MODE, IDX>(a, b, w, G); break;
-    case 8 * 4 + 0: u2_dispatch<4, 0, MODE, IDX>(a, b, w, G); break;
-    case 8 * 4 + 1: u2_dispatch<4, 1, MODE, IDX>(a, b, w, G); break;
-    case 8 * 4 + 2: u2_dispatch<4, 2, MODE, IDX>(a, b, w, G); break;
-    default: u2_dispatch<4, 3, MODE, IDX>(a, b, w, G); break;
+    red_switch<IDX, X + 1>(xr, a, w, G, acc, nred);
   }
 }
 
@@ -1262,9 +893,9 @@ __device__ __forceinline__ void jprot(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw
 template <int XR, uint32_t ACT, uint32_t SM, uint32_t KP, int MODE, typename IDX>
 __device__ __forceinline__ void jpgrp(float2 (&a)[NSLOT], float2 (&b)[NSLOT], cw_t w,
                                       const PhaseGeo<IDX>& G, IDX z0) {
-  pgrp_apply1<XR, true, ACT, SM, KP, IDX>(a, G, z0, 0u, 0u, 0u, w + PG_HDR);
+  pgrp_apply1<XR, ACT, SM, KP, IDX>(a, G, z0, w + PG_HDR);
   if constexpr (MODE == MODE_DUAL)
-    pgrp_apply1<XR, true, ACT, SM, KP, IDX>(b, G, z0, 0u, 0u, 0u, w + PG_HDR);
+    pgrp_apply1<XR, ACT, SM, KP, IDX>(b, G, z0, w + PG_HDR);
 }
 
 template <int NWAVE, int NRED>

@@ -653,7 +653,7 @@ int run_expval(tqsv_ham* h, const float2* psi, hipStream_t st) {
     if (pp.jit_fn)
       TQSV_HIP(jit_launch(pp, pl, st));
     else
-      TQSV_HIP(launch_pass(pp.tb, MODE_RED, n > 32, false, pl, st));
+      TQSV_HIP(launch_pass(pp.tb, MODE_RED, n > 32, pl, st));
     TQSV_HIP(k_final_sum(h->dpartials, pp.grid, pp.nred, h->dout + pp.red_base, st));
   }
   if (!h->small_terms.empty())
@@ -675,7 +675,7 @@ int run_expval(tqsv_ham* h, const float2* psi, hipStream_t st) {
 namespace tqsv {
 
 int plan_upload(uint32_t** dptr, size_t* cap, const std::vector<uint32_t>& prog, hipStream_t st) {
-  const size_t need = std::max<size_t>(prog.size(), 1);
+  const size_t need = prog.size() + STEP_SLACK;
   if (*cap < need) {
     if (*dptr) TQSV_HIP(hipFree(*dptr));
     *dptr = nullptr;
@@ -1224,7 +1224,6 @@ int tqsv_batch_adjoint(tqsv_batch* b, int nreq, tqsv_plan* const* plans, tqsv_ha
       return fail(TQSV_EINVAL, "tqsv_batch_adjoint: NULL argument");
     if (nreq == 0) return 0;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    bool lean = true;
     uint32_t max_nred = 0;
     size_t noff = 0, nout = 0;
     for (int i = 0; i < nreq; ++i) {
@@ -1245,7 +1244,6 @@ int tqsv_batch_adjoint(tqsv_batch* b, int nreq, tqsv_plan* const* plans, tqsv_ha
           if (!pp.tile || pp.tb != BATCH_QUBITS - RB)
             return fail(TQSV_EUNSUPPORTED, "tqsv_batch_adjoint: a plan has a pass that is not "
                                            "a whole-state tile pass");
-          lean = lean && pp.lean;
           max_nred = std::max(max_nred, pp.nred);
         }
       noff += p->passes.size() + 2 * p->rpasses.size();
@@ -1290,7 +1288,7 @@ int tqsv_batch_adjoint(tqsv_batch* b, int nreq, tqsv_plan* const* plans, tqsv_ha
                             hipMemcpyHostToDevice, st));
     TQSV_HIP(hipMemcpyAsync(b->ditems, items.data(), items.size() * sizeof(BatchItem),
                             hipMemcpyHostToDevice, st));
-    TQSV_HIP(k_batch_adjoint(b->ditems, (uint32_t)nreq, lean, max_nred, st));
+    TQSV_HIP(k_batch_adjoint(b->ditems, (uint32_t)nreq, max_nred, st));
     std::vector<double> hout(nout);
     TQSV_HIP(hipMemcpyAsync(hout.data(), b->dout, nout * sizeof(double), hipMemcpyDeviceToHost, st));
     TQSV_HIP(hipStreamSynchronize(st));

@@ -29,13 +29,15 @@ struct PassLaunch {
   double* partials;       // grid * nred doubles (reduction passes)
   uint32_t ntiles;
   uint32_t grid;
-  size_t lds_bytes;
+  uint32_t nred = 0;      // reduction slots of the pass
+  size_t lds_bytes;       // of expectation passes and generated kernels
 };
 // mode: MODE_GATE / MODE_RED / MODE_DUAL (tqsv_prog.h)
-// lean: the pass has no OP_U2 / OP_PROT steps (smaller kernel variant)
-hipError_t launch_pass(int tb, int mode, bool idx64, bool lean, const PassLaunch& pl,
-                       hipStream_t st);
+hipError_t launch_pass(int tb, int mode, bool idx64, const PassLaunch& pl, hipStream_t st);
+// LDS of expectation passes and generated kernels (2^tb threads), and of the
+// interpreting gate and dual passes (tqsv_interp.h)
 size_t pass_lds_bytes(int tb, int mode, uint32_t nred);
+size_t interp_lds_bytes(int tb, int mode, uint32_t nred);
 bool pass_variant_exists(int tb, int mode, bool idx64);
 
 // ---- single-op kernels (tqsv_kernels.hip) ----
@@ -156,7 +158,7 @@ struct BatchItem {
   double* out;             // reduction slots [0, nred), energy (re, im) at [nred, nred + 1]
   uint32_t nred;
 };
-hipError_t k_batch_adjoint(const BatchItem* items, uint32_t nreq, bool lean, uint32_t max_pass_nred,
+hipError_t k_batch_adjoint(const BatchItem* items, uint32_t nreq, uint32_t max_pass_nred,
                            hipStream_t st);
 
 }  // namespace tqsv

@@ -1,0 +1,8 @@
+// Instantiates the interpreting kernel's dual passes.
+#include "tqsv_interp.h"
+
+namespace tqsv {
+template hipError_t launch_interp<11, MODE_DUAL, uint32_t>(const PassLaunch& pl, hipStream_t st);
+template hipError_t launch_interp<12, MODE_DUAL, uint32_t>(const PassLaunch& pl, hipStream_t st);
+template hipError_t launch_interp<13, MODE_DUAL, uint32_t>(const PassLaunch& pl, hipStream_t st);
+}

@@ -1,6 +1,6 @@
-// Instantiates the tile-pass kernel for TB=8, MODE_RED, IDX=uint64_t.
+// Instantiates the expectation-pass kernel for TB=8, IDX=uint64_t.
 #include "tqsv_pass_impl.h"
 
 namespace tqsv {
-template hipError_t launch_one<8, MODE_RED, uint64_t, false>(const PassLaunch& pl, hipStream_t st);
+template hipError_t launch_one<8, uint64_t>(const PassLaunch& pl, hipStream_t st);
 }

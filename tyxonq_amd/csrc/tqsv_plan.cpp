@@ -1130,6 +1130,12 @@ int effective_tile_bits(int n, int requested, bool dual) {
   return T;
 }
 
+int plan_tile_bits(int n, const tqsv_plan_opts* opts) {
+  if (opts && opts->tile_bits > 0) return opts->tile_bits;
+  const bool interp = jit_policy(opts ? opts->jit : 0, n, 1, 1) == 0;
+  return n <= 20 && interp && !(opts && opts->min_qubits > 0) ? 12 : 13;
+}
+
 int select_passes(std::vector<Gate>& gates, const SchedOpts& so, std::vector<PassPlan>& plan) {
   const int n = so.n;
   const int T = effective_tile_bits(n, so.tile_bits, so.dual);
@@ -1143,9 +1149,10 @@ int select_passes(std::vector<Gate>& gates, const SchedOpts& so, std::vector<Pas
   const uint64_t full = lowmask(n);
   const int budget0 = so.max_cost > 0 ? so.max_cost : default_max_cost(n);
   // reduction slots per pass: the LDS beyond the tile(s) holds one double per
-  // slot and wave
-  const size_t lds_tiles = pass_lds_bytes(TBv, mode, 0);
-  const size_t nwave = ((size_t)1 << TBv) >= 64 ? ((size_t)1 << TBv) / 64 : 1;
+  // slot and wave (of the interpreting kernel, which has the most waves)
+  const size_t lds_tiles = interp_lds_bytes(TBv, mode, 0);
+  const size_t nwave = interp_lds_bytes(TBv, mode, 1) > lds_tiles
+                           ? (interp_lds_bytes(TBv, mode, 1) - lds_tiles) / sizeof(double) : 1;
   const uint32_t red_cap =
       lds_tiles < 160 * 1024 ? (uint32_t)((160 * 1024 - lds_tiles) / (nwave * sizeof(double))) : 0;
 
@@ -1409,23 +1416,14 @@ int emit_passes(std::vector<Gate>& gates, const SchedOpts& so, std::vector<PassP
     h[PH_WORDS] = (uint32_t)(prog.size() - pp.prog_off);
     for (uint32_t k = 0; k < pp.m; ++k) h[PH_H + k] = pp.H[k];
     pp.prog_words = prog.size() - pp.prog_off;
-    pp.lean = true;
-    for (size_t at = pp.prog_off + PH_SIZE, ip = 0; ip < pp.phases.size(); ++ip) {
-      const uint32_t ns = prog[at + PS_NSTEPS];
-      at += PS_SIZE;
-      for (uint32_t k = 0; k < ns; ++k) {
-        const uint32_t op = prog[at] & 0xffffu;
-        if (op == OP_U2 || op == OP_PROT || op == OP_PGRP) pp.lean = false;
-        at += prog[at] >> 16;
-      }
-    }
     pp.nred = nred;
     red_total += nred;
     pp.ntiles = (uint32_t)(1ull << (n - T));
     const uint32_t cap = nred ? 2048u : 65536u;
     pp.grid = pp.ntiles < cap ? pp.ntiles : cap;
     pp.lds = pass_lds_bytes(TBv, mode, nred);
-    if (pp.lds > 160 * 1024) return fail(TQSV_EUNSUPPORTED, "pass needs more LDS than available");
+    if (pp.lds > 160 * 1024 || interp_lds_bytes(TBv, mode, nred) > 160 * 1024)
+      return fail(TQSV_EUNSUPPORTED, "pass needs more LDS than available");
     if (!pass_variant_exists(TBv, mode, n > 32))
       return fail(TQSV_EUNSUPPORTED, "no tile-pass kernel variant for this tile size");
     passes.push_back(pp);
@@ -1525,11 +1523,12 @@ int run_passes(const std::vector<PassPlan>& passes, const std::vector<Gate>& gat
       pl.partials = part;
       pl.ntiles = pp.ntiles;
       pl.grid = pp.grid;
+      pl.nred = pp.nred;
       pl.lds_bytes = pp.lds;
       if (pp.jit_fn)
         TQSV_HIP(jit_launch(pp, pl, st));
       else
-        TQSV_HIP(launch_pass(pp.tb, pp.mode, n > 32, pp.lean, pl, st));
+        TQSV_HIP(launch_pass(pp.tb, pp.mode, n > 32, pl, st));
       if (pp.nred && !one_sum)
         TQSV_HIP(k_final_sum(dpartials, pp.grid, pp.nred, dred_out + pp.red_base, st));
     } else {

@@ -102,7 +102,6 @@ struct PassPlan {
   uint32_t ntiles = 0, grid = 0;
   size_t lds = 0;
   void* jit_fn = nullptr;  // generated kernel (hipFunction_t), when the plan uses them
-  bool lean = false;       // no OP_U2 / OP_PROT steps: the lean precompiled variant runs it
 };
 
 // Default per-pass budget (approximate VALU ops per amplitude).  Passes are
@@ -168,6 +167,14 @@ int run_passes(const std::vector<PassPlan>& passes, const std::vector<Gate>& gat
                uint32_t nslots = 0);
 
 int effective_tile_bits(int n, int requested, bool dual);
+// Tile bits of a plan that asks for none.  States of at most 20 qubits on the
+// interpreting kernel take 2^12-amplitude tiles: twice the work-groups, and two
+// waves per SIMD instead of four (energy and gradient of 8 RY/RZ/CX layers, 2^13
+// -> 2^12: 14 qubits 966 -> 818 us, 16: 1103 -> 936, 18: 1241 -> 1062, 20: 1514
+// -> 1315; the UCCSD of 16 spin orbitals 4577 -> 3639).  From 21 qubits on, 2^13
+// tiles fill the chip and fewer passes win (21 qubits 1753 against 2135 us).
+// Plans padded for batches (min_qubits) hold the whole state in one tile.
+int plan_tile_bits(int n, const tqsv_plan_opts* opts);
 
 // ---- generated pass kernels (tqsv_jit.cpp) ----
 // 1 if a plan of n qubits with the given number of tile passes uses

@@ -143,6 +143,10 @@ constexpr uint32_t RED_CROSS = 2;
 constexpr uint32_t RED_GROUP = 3;
 constexpr int RGRP_ENT = 4;
 
+// words after a program on the device: the interpreting kernel fetches the 16
+// words at the end of the last step
+constexpr int STEP_SLACK = 16;
+
 constexpr int OPH_HDR = 6;
 constexpr int OPH_ENT = 3;
 constexpr int THR_HDR = 4;
