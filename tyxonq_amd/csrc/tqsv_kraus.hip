@@ -5,7 +5,7 @@
 // Tr(K_i^dagger K_i rho), rho the qubit's 2x2 density matrix.  A chain of
 // channels is one sweep per channel: every block sums the partials that the
 // previous sweep left (all in the same order, so all choose alike), applies
-// the chosen operator to its amplitudes and accumulates the density matrix of
+// the chosen operator (times a power of two) to its amplitudes and accumulates the density matrix of
 // the next channel's qubit from the result.  Bound: one read and one write of
 // the state per channel, and launch latency below about 22 qubits.  FP64 sums.
 // 20 qubits, a trajectory of 3 layers with 20 two-operator channels each and
@@ -122,8 +122,13 @@ __global__ __launch_bounds__(BLK) void kraus_apply_kernel(float2* __restrict__ p
       }
       const double* k = k0 + 8 * (size_t)sel;
       const double w = weight(k);
-      const double f = w > 0.0 ? 1.0 / sqrt(w) : 1.0;
-      for (int j = 0; j < 8; ++j) mat[j] = (float)(f * k[j]);
+      // the nearest power of two to 1 / sqrt(w): exact, so that the operator's
+      // entries are rounded as they are given, whatever w is; the chain's last
+      // sweep normalises
+      int x = 0;
+      (void)frexp(w, &x);
+      const int e2 = w > 0.0 ? -((x - 1) >> 1) : 0;
+      for (int j = 0; j < 8; ++j) mat[j] = ldexpf((float)k[j], e2);
     }
     __syncthreads();
   }
