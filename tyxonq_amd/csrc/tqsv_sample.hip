@@ -86,12 +86,20 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(STHR) void seg_sums_kernel(const float2* __restrict__ psi,
                                                         uint32_t blk, double* __restrict__ segsum,
-                                                        double* __restrict__ bsum) {
+                                                        double* __restrict__ bsum,
+                                                        uint32_t* __restrict__ bcount,
+                                                        uint32_t* __restrict__ bfill,
+                                                        uint32_t* __restrict__ dense_n) {
   constexpr uint32_t NW = STHR / 64;
   constexpr uint32_t ROUNDS = SBLK / 128 / NW;  // wave loads of 128 amplitudes
   __shared__ double segS[SBLK / 64];
   const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
   const uint64_t base = (uint64_t)blockIdx.x * blk;
+  if (t == 0) {  // the counters of the kernels that follow
+    bcount[blockIdx.x] = 0u;
+    bfill[blockIdx.x] = 0u;
+    if (blockIdx.x == 0) *dense_n = 0u;
+  }
 #pragma unroll 4
   for (uint32_t r = 0; r < ROUNDS; ++r) {
     const uint32_t i = w * (SBLK / NW) + r * 128u + 2u * lane;
@@ -178,9 +186,54 @@ __global__ __launch_bounds__(STHR) void chunk_scan_kernel(const T* __restrict__ 
   if (lo < hi && hi == n) out[n] = run;
 }
 
-__global__ void zero_u32_kernel(uint32_t* __restrict__ p, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0u;
+// Scan of at most SCAN1 counters in one launch (whole numbers: any order of
+// the sums gives the same; the state's mass keeps its order in the three
+// launches above).  Round r of a thread holds the 4 counters at 4 (1024 r + t).
+// 16384 counters: 10 us, three launches 13 us and their gaps.
+constexpr uint32_t SROUNDS = 8;
+constexpr uint32_t SCAN1 = 4096 * SROUNDS;
+
+__global__ __launch_bounds__(1024) void scan_u32_kernel(const uint32_t* __restrict__ in, uint32_t n,
+                                                        uint32_t* __restrict__ out) {
+  __shared__ uint32_t wsum[SROUNDS][16];
+  const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+  uint32_t v[SROUNDS][4], inc[SROUNDS];
+#pragma unroll
+  for (uint32_t r = 0; r < SROUNDS; ++r)
+#pragma unroll
+    for (uint32_t u = 0; u < 4u; ++u) {
+      const uint32_t i = 4u * (1024u * r + t) + u;
+      v[r][u] = i < n ? in[i] : 0u;
+    }
+#pragma unroll
+  for (uint32_t r = 0; r < SROUNDS; ++r) {
+    inc[r] = v[r][0] + v[r][1] + v[r][2] + v[r][3];
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t u = __shfl_up(inc[r], d, 64);
+      if (lane >= (uint32_t)d) inc[r] += u;
+    }
+    if (lane == 63u) wsum[r][w] = inc[r];
+  }
+  __syncthreads();
+  uint32_t before = 0;  // the rounds before r, then the waves before this one
+#pragma unroll
+  for (uint32_t r = 0; r < SROUNDS; ++r) {
+    uint32_t pre = 0, all = 0;
+    for (uint32_t k = 0; k < 16u; ++k) {
+      if (k == w) pre = all;
+      all += wsum[r][k];
+    }
+    uint32_t run = before + pre + inc[r] - (v[r][0] + v[r][1] + v[r][2] + v[r][3]);
+    before += all;
+#pragma unroll
+    for (uint32_t u = 0; u < 4u; ++u) {
+      const uint32_t i = 4u * (1024u * r + t) + u;
+      if (i < n) out[i] = run;
+      run += v[r][u];
+    }
+  }
+  if (t == 0) out[n] = before;
 }
 
 __global__ __launch_bounds__(STHR) void shot_blocks_kernel(const double* __restrict__ prefix,
@@ -265,82 +318,97 @@ constexpr uint32_t DENSE_MIN = 32;  // blocks with more shots go to resolve_dens
 // last segment if none); the amplitude is the first lane l with
 // E[s] + (p_0 + .. + p_l) > x in that segment (lane 63 if none), moved down
 // over zero probabilities.  Only the segments that shots land in are read.
-// The LDS histogram is zeroed per 64-entry word on first use, and only the
-// touched words are compacted.
+// Bound: the latency of those scattered reads, so four shots' segments are
+// requested at a time, and the wave holds no LDS (a histogram of the block left
+// 9 waves per CU): lane j keeps the amplitude of shot j, and equal ones are
+// counted and ranked by comparing all lanes.  10^5 shots over 16384 blocks:
+// 92 -> 42 us.
 __device__ __forceinline__ double seg_prob(const float2* __restrict__ psi, uint64_t base,
                                            uint32_t blk, uint32_t i) {
   return i < blk ? prob(psi[base + i]) : 0.0;
 }
 
-__global__ __launch_bounds__(64) void resolve_kernel(const float2* __restrict__ psi, uint32_t blk,
-                                                     const double* __restrict__ segsum,
-                                                     const uint32_t* __restrict__ boff,
-                                                     const double* __restrict__ bx,
-                                                     uint64_t* __restrict__ oidx,
-                                                     uint32_t* __restrict__ ocnt,
-                                                     uint32_t* __restrict__ nuniq,
-                                                     uint32_t* __restrict__ dense_list,
-                                                     uint32_t* __restrict__ dense_n) {
-  constexpr uint32_t NWORD = SBLK / 64;
-  __shared__ uint32_t cnt[SBLK];
-  __shared__ uint64_t touched[NWORD];
-  const uint32_t b = blockIdx.x, lane = threadIdx.x;
-  const uint32_t s0 = boff[b], s1 = boff[b + 1];
-  if (s1 - s0 > DENSE_MIN) {  // left to resolve_dense_kernel
+__global__ __launch_bounds__(STHR) void resolve_kernel(const float2* __restrict__ psi, uint32_t blk,
+                                                       uint32_t nb,
+                                                       const double* __restrict__ segsum,
+                                                       const uint32_t* __restrict__ boff,
+                                                       const double* __restrict__ bx,
+                                                       uint64_t* __restrict__ oidx,
+                                                       uint32_t* __restrict__ ocnt,
+                                                       uint32_t* __restrict__ nuniq,
+                                                       uint32_t* __restrict__ dense_list,
+                                                       uint32_t* __restrict__ dense_n) {
+  constexpr uint32_t NSEG = SBLK / 64, GRP = 4;  // (8: 49 us)
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t b = __builtin_amdgcn_readfirstlane(blockIdx.x * (STHR / 64) + (threadIdx.x >> 6));
+  if (b >= nb) return;
+  const uint32_t s0 = boff[b], ns = boff[b + 1] - s0;
+  if (ns > DENSE_MIN) {  // left to resolve_dense_kernel
     if (lane == 0) dense_list[atomicAdd(dense_n, 1u)] = b;
     return;
   }
-  if (s0 == s1) {
+  if (ns == 0) {
     if (lane == 0) nuniq[b] = 0;
     return;
   }
   const uint64_t base = (uint64_t)b * blk;
   const double S = segsum[(uint64_t)b * 64u + lane];
+  const double xl = lane < ns ? bx[s0 + lane] : 0.0;  // lane j: shot j
   const double inc = wave_incl_scan_d(S, lane);
   const double ex = shfl_up_d(inc, 1);
   const double E = lane ? ex : 0.0;
   const double I = E + S;
-  touched[lane] = 0ull;
-  for (uint32_t j = s0; j < s1; ++j) {
-    const double x = bx[j];
-    const uint64_t m1 = __ballot(I > x);
-    const uint32_t seg = m1 ? (uint32_t)__builtin_ctzll(m1) : NWORD - 1u;
-    const double Es = __shfl(E, (int)seg, 64);
-    const double p = seg_prob(psi, base, blk, seg * 64u + lane);
-    const double c = Es + wave_incl_scan_d(p, lane);
-    const uint64_t m2 = __ballot(c > x);
-    const uint32_t l = m2 ? (uint32_t)__builtin_ctzll(m2) : 63u;
-    const uint64_t upto = l == 63u ? ~0ull : ((2ull << l) - 1ull);
-    const uint64_t nz = __ballot(p != 0.0) & upto;
-    uint32_t k;
-    if (nz) {
-      k = seg * 64u + (63u - (uint32_t)__builtin_clzll(nz));
-    } else {
-      k = seg * 64u;
-      while (k > 0u) {
-        --k;
-        if (seg_prob(psi, base, blk, k) != 0.0) break;
+  uint32_t mine = 0;  // lane j: the amplitude of shot j
+  for (uint32_t j0 = 0; j0 < ns; j0 += GRP) {
+    uint32_t seg[GRP];
+    double p[GRP];
+#pragma unroll
+    for (uint32_t u = 0; u < GRP; ++u) {
+      // beyond the last shot: that shot again, not kept
+      const double x = __shfl(xl, (int)min(j0 + u, ns - 1u), 64);
+      const uint64_t m1 = __ballot(I > x);
+      seg[u] = m1 ? (uint32_t)__builtin_ctzll(m1) : NSEG - 1u;
+      p[u] = seg_prob(psi, base, blk, seg[u] * 64u + lane);
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < GRP; ++u) {
+      const double x = __shfl(xl, (int)min(j0 + u, ns - 1u), 64);
+      const double Es = __shfl(E, (int)seg[u], 64);
+      const double c = Es + wave_incl_scan_d(p[u], lane);
+      const uint64_t m2 = __ballot(c > x);
+      const uint32_t l = m2 ? (uint32_t)__builtin_ctzll(m2) : 63u;
+      const uint64_t upto = l == 63u ? ~0ull : ((2ull << l) - 1ull);
+      const uint64_t nz = __ballot(p[u] != 0.0) & upto;
+      uint32_t k;
+      if (nz) {
+        k = seg[u] * 64u + (63u - (uint32_t)__builtin_clzll(nz));
+      } else {
+        k = seg[u] * 64u;
+        while (k > 0u) {
+          --k;
+          if (seg_prob(psi, base, blk, k) != 0.0) break;
+        }
       }
-    }
-    const uint32_t word = k >> 6;
-    if (touched[word] == 0ull) cnt[word * 64u + lane] = 0u;
-    if (lane == 0) {
-      cnt[k] += 1u;
-      touched[word] |= 1ull << (k & 63u);
+      if (lane == j0 + u) mine = k;
     }
   }
-  uint32_t running = 0;
-  for (uint32_t r = 0; r < NWORD; ++r) {
-    const uint64_t tw = touched[r];
-    if (!tw) continue;
-    if ((tw >> lane) & 1ull) {
-      const uint32_t pos = s0 + running + (uint32_t)__popcll(tw & ((1ull << lane) - 1ull));
-      oidx[pos] = base + r * 64u + lane;
-      ocnt[pos] = cnt[r * 64u + lane];
-    }
-    running += (uint32_t)__popcll(tw);
+  // shots of the same amplitude, and whether an earlier lane holds it
+  uint32_t same = 0;
+  bool first = lane < ns;
+  for (uint32_t i = 0; i < ns; ++i) {
+    const bool eq = (uint32_t)__shfl((int)mine, (int)i, 64) == mine;
+    same += eq ? 1u : 0u;
+    first = first && !(eq && i < lane);
   }
-  if (lane == 0) nuniq[b] = running;
+  const uint64_t fm = __ballot(first);
+  uint32_t rank = 0;
+  for (uint64_t f = fm; f; f &= f - 1ull)
+    rank += (uint32_t)__shfl((int)mine, __builtin_ctzll(f), 64) < mine ? 1u : 0u;
+  if (first) {
+    oidx[s0 + rank] = base + mine;
+    ocnt[s0 + rank] = same;
+  }
+  if (lane == 0) nuniq[b] = (uint32_t)__popcll(fm);
 }
 
 // Blocks with more than DENSE_MIN shots: the same rule, with the block's
@@ -429,14 +497,26 @@ __global__ __launch_bounds__(STHR) void resolve_dense_kernel(
   }
 }
 
+// mass and number of distinct states, in front of the results
+struct SampleHead {
+  double total;
+  uint64_t nuniq;
+};
+
 // gather the per-block (index, count) runs contiguously
 __global__ __launch_bounds__(STHR) void compact_kernel(const uint32_t* __restrict__ boff,
                                                        const uint32_t* __restrict__ uoff,
                                                        const uint64_t* __restrict__ oidx,
                                                        const uint32_t* __restrict__ ocnt,
                                                        uint64_t* __restrict__ fidx,
-                                                       int64_t* __restrict__ fcnt) {
+                                                       int64_t* __restrict__ fcnt,
+                                                       const double* __restrict__ total,
+                                                       SampleHead* __restrict__ head) {
   const uint32_t b = blockIdx.x;
+  if (b == 0 && threadIdx.x == 0) {
+    head->total = *total;
+    head->nuniq = uoff[gridDim.x];
+  }
   const uint32_t s0 = boff[b], u0 = uoff[b], nu = uoff[b + 1] - uoff[b];
   for (uint32_t k = threadIdx.x; k < nu; k += STHR) {
     fidx[u0 + k] = oidx[s0 + k];
@@ -468,6 +548,7 @@ struct tqsv_sampler {
   uint32_t* ocnt = nullptr;    // max_shots
   uint64_t* fidx = nullptr;    // max_shots
   int64_t* fcnt = nullptr;     // max_shots
+  tqsv::SampleHead* head = nullptr;
   double* csum_d = nullptr;    // chunk sums / prefixes of the scans
   double* cpre_d = nullptr;
   uint32_t* csum_u = nullptr;
@@ -480,7 +561,8 @@ void free_sampler(tqsv_sampler* s) {
   if (!s) return;
   void* ptrs[] = {s->bsum, s->segsum, s->prefix, s->bcount, s->boff, s->bfill, s->nuniq, s->uoff,
                   s->sblock, s->sx, s->bx, s->oidx, s->ocnt, s->fidx, s->fcnt,
-                  s->csum_d, s->cpre_d, s->csum_u, s->cpre_u, s->dlist, s->dn};
+                  s->csum_d, s->cpre_d, s->csum_u, s->cpre_u, s->dlist, s->dn,
+                  s->head};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete s;
@@ -501,6 +583,13 @@ hipError_t scan(const T* in, uint32_t n, T* out, T* csum, T* cpre, hipStream_t s
   hipLaunchKernelGGL(chunk_sums_kernel<T>, dim3(nc), dim3(STHR), 0, st, in, n, csum);
   hipLaunchKernelGGL(scan_kernel<T>, dim3(1), dim3(1024), 0, st, csum, nc, cpre);
   hipLaunchKernelGGL(chunk_scan_kernel<T>, dim3(nc), dim3(STHR), 0, st, in, n, cpre, out);
+  return hipGetLastError();
+}
+
+// exclusive scan of the per-block counters `in` into out[0..nb]
+hipError_t scan_counts(const tqsv_sampler* s, const uint32_t* in, uint32_t* out, hipStream_t st) {
+  if (s->nb > tqsv::SCAN1) return scan<uint32_t>(in, s->nb, out, s->csum_u, s->cpre_u, st);
+  hipLaunchKernelGGL(tqsv::scan_u32_kernel, dim3(1), dim3(1024), 0, st, in, s->nb, out);
   return hipGetLastError();
 }
 
@@ -545,6 +634,7 @@ int tqsv_sampler_create(int n, int64_t max_shots, tqsv_sampler** out) {
   if (e == hipSuccess) e = dalloc(&s->ocnt, m);
   if (e == hipSuccess) e = dalloc(&s->fidx, m);
   if (e == hipSuccess) e = dalloc(&s->fcnt, m);
+  if (e == hipSuccess) e = dalloc(&s->head, 1);
   if (e == hipSuccess) e = dalloc(&s->csum_d, nchunks(s->nb));
   if (e == hipSuccess) e = dalloc(&s->cpre_d, nchunks(s->nb) + 1);
   if (e == hipSuccess) e = dalloc(&s->csum_u, nchunks(s->nb));
@@ -571,44 +661,52 @@ int tqsv_sampler_run(tqsv_sampler* s, const void* psi, int64_t shots, uint64_t s
     const float2* a = reinterpret_cast<const float2*>(psi);
     const uint32_t nb = s->nb;
     const uint64_t ns = (uint64_t)shots;
-    const uint32_t zg = (nb + 255u) / 256u;
     hipLaunchKernelGGL(seg_sums_kernel, dim3(nb), dim3(STHR), 0, st, a, s->blk, s->segsum,
-                       s->bsum);
+                       s->bsum, s->bcount, s->bfill, s->dn);
     TQSV_HIP(hipGetLastError());
     TQSV_HIP(scan<double>(s->bsum, nb, s->prefix, s->csum_d, s->cpre_d, st));
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(zg), dim3(256), 0, st, s->bcount, nb);
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(zg), dim3(256), 0, st, s->bfill, nb);
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(256), 0, st, s->dn, 1u);
-    TQSV_HIP(hipGetLastError());
     const uint64_t ng = (ns + 3u) / 4u;
     hipLaunchKernelGGL(shot_blocks_kernel, dim3((uint32_t)((ng + STHR - 1) / STHR)), dim3(STHR), 0,
                        st, s->prefix, nb, ns, seed, (uint64_t)0, s->sblock, s->sx, s->bcount);
     TQSV_HIP(hipGetLastError());
-    TQSV_HIP(scan<uint32_t>(s->bcount, nb, s->boff, s->csum_u, s->cpre_u, st));
+    TQSV_HIP(scan_counts(s, s->bcount, s->boff, st));
     hipLaunchKernelGGL(scatter_kernel, dim3((uint32_t)((ns + 255u) / 256u)), dim3(256), 0, st,
                        s->sblock, s->sx, ns, s->boff, s->bfill, s->bx);
     TQSV_HIP(hipGetLastError());
-    hipLaunchKernelGGL(resolve_kernel, dim3(nb), dim3(64), 0, st, a, s->blk, s->segsum, s->boff,
+    hipLaunchKernelGGL(resolve_kernel, dim3((nb + STHR / 64 - 1) / (STHR / 64)), dim3(STHR), 0, st,
+                       a, s->blk, nb, s->segsum, s->boff,
                        s->bx, s->oidx, s->ocnt, s->nuniq, s->dlist, s->dn);
     hipLaunchKernelGGL(resolve_dense_kernel, dim3(std::min<uint32_t>(nb, 512u)), dim3(STHR), 0, st,
                        a, s->blk, s->segsum, s->boff, s->bx, s->oidx, s->ocnt, s->nuniq, s->dlist,
                        s->dn);
     TQSV_HIP(hipGetLastError());
-    TQSV_HIP(scan<uint32_t>(s->nuniq, nb, s->uoff, s->csum_u, s->cpre_u, st));
+    TQSV_HIP(scan_counts(s, s->nuniq, s->uoff, st));
     hipLaunchKernelGGL(compact_kernel, dim3(nb), dim3(STHR), 0, st, s->boff, s->uoff, s->oidx,
-                       s->ocnt, s->fidx, s->fcnt);
+                       s->ocnt, s->fidx, s->fcnt, s->prefix + nb, s->head);
     TQSV_HIP(hipGetLastError());
-    double total = 0.0;
-    uint32_t nu = 0;
-    TQSV_HIP(hipMemcpyAsync(&total, s->prefix + nb, sizeof(double), hipMemcpyDeviceToHost, st));
-    TQSV_HIP(hipMemcpyAsync(&nu, s->uoff + nb, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    SampleHead head{};
+    TQSV_HIP(hipMemcpyAsync(&head, s->head, sizeof(head), hipMemcpyDeviceToHost, st));
+    // a result of at most 2 MiB, if every shot is a state of its own, comes back
+    // whole with the head: one round trip instead of two (entries beyond the
+    // distinct states are not results)
+    const uint64_t most = std::min<uint64_t>(ns, s->n < 32 ? 1ull << s->n : ns);
+    const bool once = most <= (1u << 17);
+    auto fetch = [&](uint64_t k) -> int {
+      TQSV_HIP(hipMemcpyAsync(index, s->fidx, k * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+      TQSV_HIP(hipMemcpyAsync(count, s->fcnt, k * sizeof(int64_t), hipMemcpyDeviceToHost, st));
+      return 0;
+    };
+    int rc = once ? fetch(most) : 0;
+    if (rc) return rc;
     TQSV_HIP(hipStreamSynchronize(st));
-    if (!(total > 0.0) || !std::isfinite(total))
+    if (!(head.total > 0.0) || !std::isfinite(head.total))
       return fail(TQSV_EINVAL, "tqsv_sampler_run: the state has zero or non-finite norm");
-    if (nu > ns) return fail(TQSV_EDEVICE, "tqsv_sampler_run: inconsistent histogram");
-    TQSV_HIP(hipMemcpyAsync(index, s->fidx, nu * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
-    TQSV_HIP(hipMemcpyAsync(count, s->fcnt, nu * sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    TQSV_HIP(hipStreamSynchronize(st));
+    const uint64_t nu = head.nuniq;
+    if (nu > most) return fail(TQSV_EDEVICE, "tqsv_sampler_run: inconsistent histogram");
+    if (!once) {
+      if ((rc = fetch(nu))) return rc;
+      TQSV_HIP(hipStreamSynchronize(st));
+    }
     *nunique = (int64_t)nu;
     return 0;
   } catch (const std::bad_alloc&) {
