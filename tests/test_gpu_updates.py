@@ -1,0 +1,106 @@
+"""Parameter updates and coefficient changes that are queued, not waited for:
+many in flight on two streams, uses on another stream, and under capture."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+N, LAYERS = 14, 6
+
+
+def _rows(seed):
+    import tyxonq_amd as tq
+    from tyxonq_amd.engine import lower
+
+    rng = np.random.default_rng(seed)
+    c = tq.Circuit(N)
+    for _ in range(LAYERS):
+        for q in range(N):
+            c.ry(q, float(rng.normal())).rz(q, float(rng.normal()))
+        for q in range(N):
+            c.cx(q, (q + 1) % N)
+    return lower(c, mode="state")[0].segments[0][1]
+
+
+def _fresh(seed):
+    from tyxonq_amd import _native as nat
+
+    psi = nat.new_state(N, 0)
+    nat.Plan(N, _rows(seed)).run(psi)
+    return psi
+
+
+def _ham(scale):
+    from tyxonq_amd import _native as nat
+    from tyxonq_amd.pauli import PauliSum
+
+    # 8 or more diagonal terms: the diagonal vector is rebuilt with new coefficients
+    terms = [(1.0, [("Z", i), ("Z", (i + 1) % N)]) for i in range(N)] + \
+        [(1.0, [("X", i)]) for i in range(N)]
+    x, z, c = PauliSum(N, terms).to_masks()
+    return nat.Ham(N, x, z, scale * np.linspace(0.5, 1.5, len(c))), len(c)
+
+
+def test_many_updates_in_flight(gpu):
+    """More program bytes than the staging ring holds, on two streams."""
+    import torch
+
+    from tyxonq_amd import _native as nat
+
+    plans = [nat.Plan(N, _rows(0)) for _ in range(2)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    outs = []
+    for k in range(120):
+        with torch.cuda.stream(streams[k % 2]):
+            psi = nat.new_state(N, 0)
+            plans[k % 2].update(_rows(k % 7))
+            plans[k % 2].run(psi)
+            outs.append(psi)
+    torch.cuda.synchronize()
+    ref = [_fresh(s) for s in range(7)]
+    for k, psi in enumerate(outs):
+        assert torch.equal(psi, ref[k % 7])
+
+
+def test_update_used_on_another_stream_and_under_capture(gpu):
+    import torch
+
+    from tyxonq_amd import _native as nat
+
+    plan = nat.Plan(N, _rows(1))
+    ham, nt = _ham(1.0)
+    psi, out = nat.new_state(N, 0), nat.new_state(N, 0)
+    want = torch.empty_like(out)
+    ham2, _ = _ham(-2.0)
+    ham2.apply(_fresh(2), want)
+
+    def go():
+        nat.init_basis(psi, 0)
+        plan.run(psi)
+        ham.apply(psi, out)
+
+    go()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    plan.update(_rows(2))
+    ham.set_coeffs(-2.0 * np.linspace(0.5, 1.5, nt))
+    with torch.cuda.stream(side):
+        go()
+    side.synchronize()
+    assert torch.equal(out, want)
+    plan.update(_rows(2))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        go()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        psi.normal_()  # eager work between the replays
+    with pytest.raises(NotImplementedError):
+        with torch.cuda.graph(torch.cuda.CUDAGraph()):
+            plan.update(_rows(3))

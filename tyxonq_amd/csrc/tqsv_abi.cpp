@@ -560,6 +560,8 @@ int tqsv_plan_create(int n, const tqsv_op* ops, int nops, const tqsv_plan_opts* 
     p->jit_req = opts ? opts->jit : 0;
     const int rc = plan_build_forward(p.get(), ops, nops, nullptr);
     if (rc) return rc;
+    TQSV_HIP(hipStreamSynchronize(nullptr));
+    p->uploaded.clear();
     *out = p.release();
     return 0;
   } catch (const std::bad_alloc&) {
@@ -689,6 +691,7 @@ int tqsv_plan_precompile(int n, const tqsv_op* ops, int nops, const tqsv_plan_op
 int tqsv_plan_run(tqsv_plan* p, void* psi, void* stream) {
   if (!p || !psi) return fail(TQSV_EINVAL, "tqsv_plan_run: NULL argument");
   hipStream_t st = S(stream);
+  TQSV_HIP(p->uploaded.wait(st));
   if (p->n == p->nu)
     return run_passes(p->passes, p->gates, p->n, p->dprog, F(psi), nullptr, nullptr, nullptr, st);
   TQSV_HIP(k_pad_copy(F(psi), 1ull << p->nu, p->pad_a, 1ull << p->n, st));

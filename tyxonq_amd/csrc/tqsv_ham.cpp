@@ -90,6 +90,7 @@ struct tqsv_ham {
   float* d_diag = nullptr;
   uint64_t* d_dz = nullptr;
   double* d_dc = nullptr;
+  tqsv::StreamMark uploaded;     // the last coefficient copies and d_diag's kernel
   bool jit_ready = false;        // generated expectation kernels compiled
 
   ~tqsv_ham() {
@@ -441,13 +442,13 @@ std::vector<float2> sub_tables(const tqsv_ham* h) {
   return tab;
 }
 
-// the diagonal vector from the current coefficients (on stream st, waited for)
+// queues the diagonal vector of the current coefficients
 int build_diag(tqsv_ham* h, hipStream_t st) {
   std::vector<double> dc;
   for (int t : h->diag_terms) dc.push_back(h->coeff[t]);
-  TQSV_HIP(hipMemcpyAsync(h->d_dc, dc.data(), dc.size() * sizeof(double), hipMemcpyHostToDevice, st));
+  const int rc = stage_copy(h->d_dc, dc.data(), dc.size() * sizeof(double), st);
+  if (rc) return rc;
   TQSV_HIP(k_diag_build(h->d_diag, h->n, (uint32_t)dc.size(), h->d_dz, h->d_dc, st));
-  TQSV_HIP(hipStreamSynchronize(st));
   return 0;
 }
 
@@ -608,6 +609,7 @@ int plan_apply(tqsv_ham* h) {
     TQSV_HIP(hipMalloc(reinterpret_cast<void**>(&h->d_diag), sizeof(float) << h->n));
     const int rc = build_diag(h, nullptr);
     if (rc) return rc;
+    TQSV_HIP(hipStreamSynchronize(nullptr));
   }
   return 0;
 }
@@ -682,12 +684,7 @@ int plan_upload(uint32_t** dptr, size_t* cap, const std::vector<uint32_t>& prog,
     TQSV_HIP(hipMalloc(reinterpret_cast<void**>(dptr), need * sizeof(uint32_t)));
     *cap = need;
   }
-  if (!prog.empty()) {
-    TQSV_HIP(hipMemcpyAsync(*dptr, prog.data(), prog.size() * sizeof(uint32_t),
-                            hipMemcpyHostToDevice, st));
-    TQSV_HIP(hipStreamSynchronize(st));
-  }
-  return 0;
+  return stage_copy(*dptr, prog.data(), prog.size() * sizeof(uint32_t), st);
 }
 
 static size_t count_tile(const std::vector<PassPlan>& passes) {
@@ -759,7 +756,11 @@ int plan_build_forward(tqsv_plan* p, const tqsv_op* ops, int nops, hipStream_t s
   p->passes.swap(passes);
   p->prog.swap(prog);
   p->adj_built = false;
-  return plan_upload(&p->dprog, &p->dprog_cap, p->prog, st);
+  TQSV_HIP(p->uploaded.wait(st));  // an earlier copy on another stream
+  rc = plan_upload(&p->dprog, &p->dprog_cap, p->prog, st);
+  if (rc) return rc;
+  TQSV_HIP(p->uploaded.record(st));
+  return 0;
 }
 
 // grow *d to `need` doubles keeping its first `keep`: work queued on st may
@@ -907,8 +908,13 @@ int plan_build_adjoint(tqsv_plan* p, hipStream_t st) {
   if (pcap >= (1ull << 32)) return fail(TQSV_EINVAL, "reverse sweep: too many reduction partials");
   rc = plan_upload(&p->drprog, &p->drprog_cap, p->rprog, st);
   if (rc) return rc;
-  rc = plan_upload(&p->dslots, &p->dslots_cap, p->hslots, st);
-  if (rc) return rc;
+  if (p->uslots != p->hslots) {  // fixed by the program's structure
+    p->uslots.clear();
+    rc = plan_upload(&p->dslots, &p->dslots_cap, p->hslots, st);
+    if (rc) return rc;
+    p->uslots = p->hslots;
+  }
+  TQSV_HIP(p->uploaded.record(st));
   // the energy partials of a queued H|psi> may already be in the buffer
   rc = grow_keep(&p->dpartials, &p->dpartials_cap, pcap, 2 * (size_t)eg, st);
   if (rc) return rc;
@@ -1096,13 +1102,13 @@ int tqsv_ham_set_coeffs(tqsv_ham* h, int nterms, const double* coeff, void* stre
     const std::vector<float2> rtc = apply_coeffs(h, h->rest_order);
     const std::vector<float2> tab = sub_tables(h);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    TQSV_HIP(hipMemcpyAsync(h->d_tc, tc.data(), tc.size() * sizeof(float2), hipMemcpyHostToDevice, st));
-    if (!rtc.empty())
-      TQSV_HIP(hipMemcpyAsync(h->d_rtc, rtc.data(), rtc.size() * sizeof(float2), hipMemcpyHostToDevice, st));
-    if (!tab.empty())
-      TQSV_HIP(hipMemcpyAsync(h->d_stab, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice, st));
-    TQSV_HIP(hipStreamSynchronize(st));
-    if (!h->diag_terms.empty()) return build_diag(h, st);
+    TQSV_HIP(h->uploaded.wait(st));
+    int rc = stage_copy(h->d_tc, tc.data(), tc.size() * sizeof(float2), st);
+    if (!rc) rc = stage_copy(h->d_rtc, rtc.data(), rtc.size() * sizeof(float2), st);
+    if (!rc) rc = stage_copy(h->d_stab, tab.data(), tab.size() * sizeof(float2), st);
+    if (!rc && !h->diag_terms.empty()) rc = build_diag(h, st);
+    if (rc) return rc;
+    TQSV_HIP(h->uploaded.record(st));
     return 0;
   } catch (const std::bad_alloc&) {
     return fail(TQSV_ENOMEM, "tqsv_ham_set_coeffs: out of host memory");
@@ -1128,6 +1134,7 @@ int tqsv_ham_expval(tqsv_ham* h, const void* psi, double* terms, double* energy,
 int tqsv_ham_apply(tqsv_ham* h, const void* psi, void* out, void* stream) {
   if (!h || !psi || !out) return fail(TQSV_EINVAL, "tqsv_ham_apply: NULL argument");
   if (psi == out) return fail(TQSV_EINVAL, "tqsv_ham_apply: out must not alias psi");
+  TQSV_HIP(h->uploaded.wait(reinterpret_cast<hipStream_t>(stream)));
   TQSV_HIP(k_ham_apply(reinterpret_cast<const float2*>(psi), reinterpret_cast<float2*>(out), h->n,
                        h->apply_args(), reinterpret_cast<hipStream_t>(stream)));
   return 0;
@@ -1185,8 +1192,10 @@ int tqsv_adjoint(tqsv_plan* p, tqsv_ham* h, void* psi, void* lam, int nparams, d
       TQSV_HIP(k_pad_copy(reinterpret_cast<const float2*>(psi), 1ull << p->nu, a, 1ull << p->n, st));
       TQSV_HIP(k_pad_copy(nullptr, 0, b, 1ull << p->n, st));
     }
+    TQSV_HIP(p->uploaded.wait(st));
     rc = run_passes(p->passes, p->gates, p->n, p->dprog, a, nullptr, nullptr, nullptr, st);
     if (rc) return rc;
+    TQSV_HIP(h->uploaded.wait(st));
     // lambda = H psi and the block partials of E = Re <psi|H psi>
     TQSV_HIP(k_ham_apply(a, b, h->n, h->apply_args(), st, p->dpartials));
     // the reverse programs are built on the host while the device runs the
@@ -1228,7 +1237,7 @@ int tqsv_batch_adjoint(tqsv_batch* b, int nreq, tqsv_plan* const* plans, tqsv_ha
     size_t noff = 0, nout = 0;
     for (int i = 0; i < nreq; ++i) {
       tqsv_plan* p = plans[i];
-      const tqsv_ham* h = hams[i];
+      tqsv_ham* h = hams[i];
       if (!p || !h || !psi[i] || (nparams[i] > 0 && !grads[i]))
         return fail(TQSV_EINVAL, "tqsv_batch_adjoint: NULL request field");
       if (p->n != BATCH_QUBITS || p->nu != h->n)
@@ -1237,6 +1246,8 @@ int tqsv_batch_adjoint(tqsv_batch* b, int nreq, tqsv_plan* const* plans, tqsv_ha
       if (nparams[i] <= p->max_param)
         return fail(TQSV_EINVAL, "tqsv_batch_adjoint: nparams smaller than the largest parameter "
                                  "index + 1");
+      TQSV_HIP(p->uploaded.wait(st));
+      TQSV_HIP(h->uploaded.wait(st));
       int rc = plan_build_adjoint(p, st);
       if (rc) return rc;
       for (const auto* v : {&p->passes, &p->rpasses})
@@ -1284,10 +1295,8 @@ int tqsv_batch_adjoint(tqsv_batch* b, int nreq, tqsv_plan* const* plans, tqsv_ha
       outpos[(size_t)i] = opos;
       opos += (size_t)p->nred_adj + 2;
     }
-    TQSV_HIP(hipMemcpyAsync(b->doff, off.data(), off.size() * sizeof(uint32_t),
-                            hipMemcpyHostToDevice, st));
-    TQSV_HIP(hipMemcpyAsync(b->ditems, items.data(), items.size() * sizeof(BatchItem),
-                            hipMemcpyHostToDevice, st));
+    if ((rc = stage_copy(b->doff, off.data(), off.size() * sizeof(uint32_t), st))) return rc;
+    if ((rc = stage_copy(b->ditems, items.data(), items.size() * sizeof(BatchItem), st))) return rc;
     TQSV_HIP(k_batch_adjoint(b->ditems, (uint32_t)nreq, max_nred, st));
     std::vector<double> hout(nout);
     TQSV_HIP(hipMemcpyAsync(hout.data(), b->dout, nout * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -1310,6 +1319,7 @@ int tqsv_vjp(tqsv_plan* p, void* psi, void* lam, int nparams, double* grad, void
       return fail(TQSV_EINVAL, "tqsv_vjp: nparams smaller than the largest parameter index + 1");
     if (psi == lam) return fail(TQSV_EINVAL, "tqsv_vjp: lam must not alias psi");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    TQSV_HIP(p->uploaded.wait(st));
     int rc = plan_build_adjoint(p, st);
     if (rc) return rc;
     std::vector<double> hred((size_t)p->nred_adj + 2);

@@ -11,6 +11,7 @@
 #include "../../include/tqsv.h"
 #include "tqsv_internal.h"
 #include "tqsv_prog.h"
+#include "tqsv_stage.h"
 
 namespace tqsv {
 
@@ -230,7 +231,7 @@ struct tqsv_plan {
   // index} (one final sum for the whole sweep), then two entries for the
   // energy of tqsv_adjoint, whose block partials (from H|psi>) lead the
   // partials buffer
-  std::vector<uint32_t> hslots;
+  std::vector<uint32_t> hslots, uslots;  // uslots: as last uploaded
   uint32_t* dslots = nullptr;
   size_t dslots_cap = 0;
   int max_param = -1;
@@ -249,6 +250,7 @@ struct tqsv_plan {
   // amplitudes are copied into pad_a (pad_b for lambda), the rest is zero.
   float2* pad_a = nullptr;
   float2* pad_b = nullptr;
+  tqsv::StreamMark uploaded;  // the last program copies
 };
 
 #endif

@@ -227,7 +227,9 @@ def execute_batch(reqs: List[Request], cache: Cache) -> List[Tuple[float, np.nda
     """Energies and gradients of small requests in one launch (current stream)."""
     got = [cache.acquire(r) for r in reqs]
     try:
-        psis = [nat.new_state(r.n, 0) for r in reqs]
+        # the launch only reads the initial states: one |0> per size
+        zero = {n: nat.new_state(n, 0) for n in {r.n for r in reqs}}
+        psis = [zero[r.n] for r in reqs]
         out = cache.get_batch().adjoint([p for p, _ in got], [h for _, h in got], psis,
                                         [len(r.params) for r in reqs])
     finally:
