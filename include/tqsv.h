@@ -231,6 +231,11 @@ int tqsv_plan_create(int n, const tqsv_op* ops, int nops, const tqsv_plan_opts* 
  * unchanged (same kinds, targets, controls, masks) and re-upload. */
 int tqsv_plan_update(tqsv_plan* plan, const tqsv_op* ops, int nops, void* stream);
 
+/* tqsv_plan_update of several plans at once: the programs are written on several
+ * host threads.  A plan may appear once. */
+int tqsv_plan_update_many(int nplans, tqsv_plan* const* plans, const tqsv_op* const* ops,
+                          const int* nops, void* stream);
+
 int tqsv_plan_get_info(const tqsv_plan* plan, tqsv_plan_info* info);
 
 /* Plan on the host only (no device memory is touched) and report what

@@ -104,3 +104,32 @@ def test_update_used_on_another_stream_and_under_capture(gpu):
     with pytest.raises(NotImplementedError):
         with torch.cuda.graph(torch.cuda.CUDAGraph()):
             plan.update(_rows(3))
+
+
+@pytest.mark.parametrize("count", [0, 1, 7, 8, 40])
+def test_update_many(gpu, count):
+    """One thread, two threads and eight; a wrong op count fails and says so."""
+    from tyxonq_amd import _native as nat
+
+    rows = [_rows(s) for s in range(5)]
+    plans = [nat.Plan(N, rows[0]) for _ in range(count)]
+    nat.update_plans(plans, [rows[(k + 1) % 5] for k in range(count)])
+    ref = [_fresh(s) for s in range(5)]
+    for k, p in enumerate(plans):
+        psi = nat.new_state(N, 0)
+        p.run(psi)
+        assert (psi == ref[(k + 1) % 5]).all()
+    if count:
+        with pytest.raises(ValueError, match="op count"):
+            nat.update_plans(plans, [r[:-1] for r in [rows[0]] * count])
+        bad = rows[1].copy()
+        bad["kind"][3] = 99
+        with pytest.raises(ValueError, match="op 3"):
+            nat.update_plans(plans, [rows[2]] * (count - 1) + [bad])
+        for k, p in enumerate(plans):  # the others are updated, the bad one is as it was
+            psi = nat.new_state(N, 0)
+            p.run(psi)
+            assert (psi == ref[2 if k < count - 1 else (k + 1) % 5]).all()
+    if count > 1:
+        with pytest.raises(ValueError, match="repeated"):
+            nat.update_plans([plans[0], plans[0]], [rows[0], rows[0]])

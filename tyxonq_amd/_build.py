@@ -43,6 +43,9 @@ CXX_FLAGS = [
     "-O2",
     "-std=c++17",
     "-fPIC",
+    # complex products without the NaN recovery of C99's Annex G (the planner's
+    # values are finite)
+    "-fcx-fortran-rules",
     "-D__HIP_PLATFORM_AMD__",
     f"-I{ROCM / 'include'}",
     "-Wall",

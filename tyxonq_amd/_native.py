@@ -122,6 +122,7 @@ _SIGS = {
     "tqsv_probs": (_I, [_P, _I, _P, _P]),
     "tqsv_plan_create": (_I, [_I, _P, _I, ctypes.POINTER(PlanOpts), ctypes.POINTER(_P)]),
     "tqsv_plan_update": (_I, [_P, _P, _I, _P]),
+    "tqsv_plan_update_many": (_I, [_I, _P, _P, _P, _P]),
     "tqsv_plan_get_info": (_I, [_P, ctypes.POINTER(PlanInfo)]),
     "tqsv_plan_inspect": (_I, [_I, _P, _I, ctypes.POINTER(PlanOpts), ctypes.POINTER(PlanInfo)]),
     "tqsv_plan_emulate": (_I, [_I, _P, _I, ctypes.POINTER(PlanOpts), _P]),
@@ -571,6 +572,23 @@ class Plan:
             self.close()
         except Exception:
             pass
+
+
+def update_plans(plans: Sequence["Plan"], ops: Sequence[np.ndarray]) -> None:
+    """Plan.update of several different plans at once (on several host threads)."""
+    k = len(plans)
+    if len(ops) != k:
+        raise ValueError("plans and ops must have equal length")
+    if k == 0:
+        return
+    rows = [np.ascontiguousarray(o, dtype=OP_DTYPE) for o in ops]
+    P = (ctypes.c_void_p * k)(*[p._h.value for p in plans])
+    O = (ctypes.c_void_p * k)(*[o.ctypes.data if len(o) else None for o in rows])
+    N = (ctypes.c_int * k)(*[len(o) for o in rows])
+    for p, o in zip(plans, rows):
+        p._ops = o
+    _check(load().tqsv_plan_update_many(k, ctypes.cast(P, _P), ctypes.cast(O, _P),
+                                        ctypes.cast(N, _P), stream_ptr()))
 
 
 class Ham:

@@ -11,12 +11,14 @@
 // LDS, per-work-group partials and a fixed-order final sum: the result does
 // not depend on launch timing.
 #include <algorithm>
+#include <atomic>
 #include <new>
 #include <cmath>
 #include <cstring>
 #include <map>
 #include <memory>
 #include <string>
+#include <thread>
 
 #include "tqsv_planner.h"
 
@@ -718,7 +720,8 @@ static int attach_kernels(std::vector<PassPlan>& passes, const std::vector<uint3
   return 0;
 }
 
-int plan_build_forward(tqsv_plan* p, const tqsv_op* ops, int nops, hipStream_t st) {
+// the host part of a forward build (with generated kernels: their compilation)
+static int plan_emit_forward(tqsv_plan* p, const tqsv_op* ops, int nops) {
   std::vector<Gate>& g = p->gwork;
   int rc = gates_from_ops(p->nu, ops, nops, g);
   if (rc) return rc;
@@ -756,10 +759,54 @@ int plan_build_forward(tqsv_plan* p, const tqsv_op* ops, int nops, hipStream_t s
   p->passes.swap(passes);
   p->prog.swap(prog);
   p->adj_built = false;
+  return 0;
+}
+
+static int plan_upload_forward(tqsv_plan* p, hipStream_t st) {
   TQSV_HIP(p->uploaded.wait(st));  // an earlier copy on another stream
-  rc = plan_upload(&p->dprog, &p->dprog_cap, p->prog, st);
+  const int rc = plan_upload(&p->dprog, &p->dprog_cap, p->prog, st);
   if (rc) return rc;
   TQSV_HIP(p->uploaded.record(st));
+  return 0;
+}
+
+int plan_build_forward(tqsv_plan* p, const tqsv_op* ops, int nops, hipStream_t st) {
+  const int rc = plan_emit_forward(p, ops, nops);
+  return rc ? rc : plan_upload_forward(p, st);
+}
+
+// f(i) for i < n, on up to 8 threads when every call is host work of tens of
+// microseconds (a batch of 48 requests of 2-13 qubits, forward and reverse
+// programs: 11.7 -> 7.6 ms in all).  Fewer than 8 calls stay on this thread (a
+// thread costs about as much as a call).  Returns the first failing call's code
+// and sets its message.
+template <typename F>
+static int parallel_calls(int n, F f) {
+  const int nt = std::min(8, std::min(n / 4, (int)std::thread::hardware_concurrency()));
+  std::vector<std::pair<int, std::string>> res((size_t)n);
+  std::atomic<int> next{0};
+  auto work = [&]() {
+    for (int i; (i = next.fetch_add(1)) < n;) {
+      auto& r = res[(size_t)i];
+      try {
+        r.first = f(i);
+        if (r.first) r.second = tqsv_last_error();
+      } catch (const std::exception& e) {
+        r.first = TQSV_ENOMEM;
+        r.second = e.what();
+      }
+    }
+  };
+  std::vector<std::thread> pool;
+  try {
+    for (int t = 1; t < nt; ++t) pool.emplace_back(work);
+  } catch (const std::exception&) {
+    // fewer threads than asked for
+  }
+  work();
+  for (std::thread& t : pool) t.join();
+  for (const auto& r : res)
+    if (r.first) return fail(r.first, r.second);
   return 0;
 }
 
@@ -840,8 +887,8 @@ void reverse_gates(const std::vector<Gate>& gates, std::vector<Gate>& r) {
   }
 }
 
-int plan_build_adjoint(tqsv_plan* p, hipStream_t st) {
-  if (p->adj_built) return 0;
+// the host part of a reverse build
+static int plan_emit_adjoint(tqsv_plan* p) {
   std::vector<Gate>& r = p->rwork;
   reverse_gates(p->gates, r);
   const bool same = same_structure(r, p->rgates) && !p->rsel.empty();
@@ -906,7 +953,12 @@ int plan_build_adjoint(tqsv_plan* p, hipStream_t st) {
   slot(red_total, 0, eg, 2, 0);
   slot(red_total + 1, 0, eg, 2, 1);
   if (pcap >= (1ull << 32)) return fail(TQSV_EINVAL, "reverse sweep: too many reduction partials");
-  rc = plan_upload(&p->drprog, &p->drprog_cap, p->rprog, st);
+  p->need_partials = pcap;
+  return 0;
+}
+
+static int plan_upload_adjoint(tqsv_plan* p, hipStream_t st) {
+  int rc = plan_upload(&p->drprog, &p->drprog_cap, p->rprog, st);
   if (rc) return rc;
   if (p->uslots != p->hslots) {  // fixed by the program's structure
     p->uslots.clear();
@@ -916,12 +968,19 @@ int plan_build_adjoint(tqsv_plan* p, hipStream_t st) {
   }
   TQSV_HIP(p->uploaded.record(st));
   // the energy partials of a queued H|psi> may already be in the buffer
-  rc = grow_keep(&p->dpartials, &p->dpartials_cap, pcap, 2 * (size_t)eg, st);
+  const uint32_t eg = ham_apply_grid(p->nu);
+  rc = grow_keep(&p->dpartials, &p->dpartials_cap, p->need_partials, 2 * (size_t)eg, st);
   if (rc) return rc;
-  rc = ensure(&p->dred, &p->dred_cap, (size_t)red_total + 2);
+  rc = ensure(&p->dred, &p->dred_cap, (size_t)p->nred_adj + 2);
   if (rc) return rc;
   p->adj_built = true;
   return 0;
+}
+
+int plan_build_adjoint(tqsv_plan* p, hipStream_t st) {
+  if (p->adj_built) return 0;
+  const int rc = plan_emit_adjoint(p);
+  return rc ? rc : plan_upload_adjoint(p, st);
 }
 
 // dE/dparam from the reverse sweep's reduction slots:
@@ -1217,6 +1276,40 @@ int tqsv_adjoint(tqsv_plan* p, tqsv_ham* h, void* psi, void* lam, int nparams, d
   }
 }
 
+int tqsv_plan_update_many(int nplans, tqsv_plan* const* plans, const tqsv_op* const* ops,
+                          const int* nops, void* stream) {
+  try {
+    if (nplans < 0 || (nplans > 0 && (!plans || !ops || !nops)))
+      return fail(TQSV_EINVAL, "tqsv_plan_update_many: NULL argument");
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    bool serial = false;
+    for (int i = 0; i < nplans; ++i) {
+      if (!plans[i]) return fail(TQSV_EINVAL, "tqsv_plan_update_many: plan is NULL");
+      if (nops[i] != plans[i]->nops)
+        return fail(TQSV_EINVAL, "tqsv_plan_update_many: op count changed");
+      if (nops[i] > 0 && !ops[i]) return fail(TQSV_EINVAL, "tqsv_plan_update_many: bad op array");
+      for (int j = 0; j < i; ++j)
+        if (plans[j] == plans[i]) return fail(TQSV_EINVAL, "tqsv_plan_update_many: repeated plan");
+      serial = serial || jit_policy(plans[i]->jit_req, plans[i]->n, 1, 64);
+    }
+    auto emit = [&](int i) { return plan_emit_forward(plans[i], ops[i], nops[i]); };
+    int rc = 0;
+    if (serial) {
+      for (int i = 0; !rc && i < nplans; ++i) rc = emit(i);
+    } else {
+      rc = parallel_calls(nplans, emit);
+    }
+    // after a failure too: the plans that were written are complete
+    for (int i = 0; i < nplans; ++i) {
+      const int r = plan_upload_forward(plans[i], st);
+      if (!rc) rc = r;
+    }
+    return rc;
+  } catch (const std::bad_alloc&) {
+    return fail(TQSV_ENOMEM, "tqsv_plan_update_many: out of host memory");
+  }
+}
+
 int tqsv_batch_create(tqsv_batch** out) {
   if (!out) return fail(TQSV_EINVAL, "tqsv_batch_create: NULL output");
   *out = new (std::nothrow) tqsv_batch();
@@ -1235,6 +1328,8 @@ int tqsv_batch_adjoint(tqsv_batch* b, int nreq, tqsv_plan* const* plans, tqsv_ha
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     uint32_t max_nred = 0;
     size_t noff = 0, nout = 0;
+    int rc = 0;
+    std::vector<tqsv_plan*> build;  // plans whose reverse programs are out of date, once each
     for (int i = 0; i < nreq; ++i) {
       tqsv_plan* p = plans[i];
       tqsv_ham* h = hams[i];
@@ -1246,10 +1341,26 @@ int tqsv_batch_adjoint(tqsv_batch* b, int nreq, tqsv_plan* const* plans, tqsv_ha
       if (nparams[i] <= p->max_param)
         return fail(TQSV_EINVAL, "tqsv_batch_adjoint: nparams smaller than the largest parameter "
                                  "index + 1");
-      TQSV_HIP(p->uploaded.wait(st));
-      TQSV_HIP(h->uploaded.wait(st));
-      int rc = plan_build_adjoint(p, st);
+      if (!p->adj_built && std::find(build.begin(), build.end(), p) == build.end()) build.push_back(p);
+    }
+    if (!build.empty()) {
+      // (generated kernels, forced by TQSV_JIT, are compiled one plan at a time)
+      auto emit = [&](int i) { return plan_emit_adjoint(build[(size_t)i]); };
+      if (jit_policy(build[0]->jit_req, BATCH_QUBITS, 1, 64)) {
+        for (int i = 0; !rc && i < (int)build.size(); ++i) rc = emit(i);
+      } else {
+        rc = parallel_calls((int)build.size(), emit);
+      }
       if (rc) return rc;
+    }
+    for (tqsv_plan* p : build) {
+      TQSV_HIP(p->uploaded.wait(st));
+      if ((rc = plan_upload_adjoint(p, st))) return rc;
+    }
+    for (int i = 0; i < nreq; ++i) {
+      tqsv_plan* p = plans[i];
+      TQSV_HIP(p->uploaded.wait(st));
+      TQSV_HIP(hams[i]->uploaded.wait(st));
       for (const auto* v : {&p->passes, &p->rpasses})
         for (const PassPlan& pp : *v) {
           if (!pp.tile || pp.tb != BATCH_QUBITS - RB)
@@ -1260,7 +1371,7 @@ int tqsv_batch_adjoint(tqsv_batch* b, int nreq, tqsv_plan* const* plans, tqsv_ha
       noff += p->passes.size() + 2 * p->rpasses.size();
       nout += (size_t)p->nred_adj + 2;
     }
-    int rc = grow(&b->doff, &b->doff_cap, noff);
+    rc = grow(&b->doff, &b->doff_cap, noff);
     if (!rc) rc = grow(&b->ditems, &b->items_cap, (size_t)nreq);
     if (!rc) rc = grow(&b->dout, &b->out_cap, nout);
     if (rc) return rc;

@@ -264,7 +264,14 @@ void block(const Gate& g, uint64_t& blkN, uint64_t& blkD) {
 constexpr double kTwoPi = 6.283185307179586476925286766559;
 constexpr double kPi = 3.1415926535897932384626433832795;
 
-inline cd wrap(cd v) { return cd(v.real(), std::remainder(v.imag(), kTwoPi)); }
+// the phase reduced to [-pi, pi]: std::remainder's exact result, which below 3 pi
+// is one exact subtraction (the operands are within a factor of two)
+inline cd wrap(cd v) {
+  const double a = std::abs(v.imag());
+  if (a <= kPi) return v;
+  if (a < 9.42) return cd(v.real(), v.imag() - std::copysign(kTwoPi, v.imag()));
+  return cd(v.real(), std::remainder(v.imag(), kTwoPi));
+}
 inline bool trivial(cd v) { return std::abs(v.real()) < 1e-14 && std::abs(v.imag()) < 1e-13; }
 // exp(v) == -1 (a sign)
 inline bool is_sign(cd v) {
@@ -273,7 +280,10 @@ inline bool is_sign(cd v) {
 inline cd cexp_snap(cd v) {
   if (trivial(v)) return cd(1, 0);
   if (is_sign(v)) return cd(-1, 0);
-  return std::exp(v);
+  if (v.real() != 0.0) return std::exp(v);
+  double sn, cs;
+  sincos(v.imag(), &sn, &cs);
+  return cd(cs, sn);
 }
 
 struct Pend {
@@ -455,15 +465,12 @@ struct Slots {
   Slots(const std::array<uint32_t, RB>& Rp, const TileGeo& geo) {
     for (int b = 0; b < 64; ++b) of_bit[b] = -1;
     for (int j = 0; j < RB; ++j) bit_of[j] = -1;
-    for (int b = 0; b < 64; ++b) {
-      const int p = geo.pos(b);
-      if (p < 0) continue;
-      for (int j = 0; j < RB; ++j)
-        if ((int)Rp[j] == p) {
-          of_bit[b] = j;
-          bit_of[j] = b;
-          reg |= bitm(b);
-        }
+    for (int j = 0; j < RB; ++j) {
+      const int p = (int)Rp[j];
+      const int b = p < geo.L ? p : geo.H[(size_t)(p - geo.L)];
+      of_bit[b] = j;
+      bit_of[j] = b;
+      reg |= bitm(b);
     }
   }
 };
@@ -521,22 +528,19 @@ struct PhaseEmitter {
       if (S.reg & bitm(ctz(u))) rr = true;
     if (rr) regreg();
     const cd U0 = cexp_snap(P.lin[q]);
-    std::vector<std::pair<int, cd>> ents;
-    for (uint64_t u = P.qm[q]; u; u &= u - 1) {
-      const int p = ctz(u);
-      ents.push_back({p, cexp_snap(P.qref(q, p))});
-    }
-    for (const auto& x : ents) P.clear_quad(q, x.first);
+    const uint64_t on = P.qm[q];
     P.clear_lin(q);
-    if (U0 == cd(1, 0) && ents.empty()) return;
+    if (U0 == cd(1, 0) && !on) return;
     const size_t at = e.begin(OP_PH);
     e.u((uint32_t)S.of_bit[q]);
-    e.u((uint32_t)ents.size());
+    e.u((uint32_t)popc(on));
     e.u(0);
     e.c(U0);
-    for (const auto& x : ents) {
-      e.u((uint32_t)x.first);
-      e.c(x.second);
+    for (uint64_t u = on; u; u &= u - 1) {
+      const int p = ctz(u);
+      e.u((uint32_t)p);
+      e.c(cexp_snap(P.qref(q, p)));
+      P.clear_quad(q, p);
     }
     e.end(at);
   }

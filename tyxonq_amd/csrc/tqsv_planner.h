@@ -223,6 +223,7 @@ struct tqsv_plan {
   uint32_t* drprog = nullptr;
   size_t drprog_cap = 0;
   int nred_adj = 0;
+  size_t need_partials = 0;  // doubles of block partials of the reverse sweep
   double* dpartials = nullptr;
   size_t dpartials_cap = 0;
   double* dred = nullptr;

@@ -196,14 +196,15 @@ class Cache:
         self.hams: Dict[Tuple[int, str], List["nat.Ham"]] = {}
         self.batch: Optional["nat.Batch"] = None
 
-    def acquire(self, req: Request):
+    def _take(self, req: Request):
+        """(plan, op rows to update it with or None, ham) of a request."""
         ops = request_ops(req)
         pool = self.plans.setdefault((req.n, req.depth), [])
         if pool:
-            plan = pool.pop()
-            plan.update(ops)
+            plan, todo = pool.pop(), ops
         else:
             plan = nat.Plan(req.n, ops, jit=-1, min_qubits=BATCH_MAX_QUBITS if is_small(req) else 0)
+            todo = None
         hpool = self.hams.setdefault((req.n, req.ham), [])
         if hpool:
             ham = hpool.pop()
@@ -211,7 +212,17 @@ class Cache:
         else:
             x, z, c = PauliSum(req.n, request_terms(req)).to_masks()
             ham = nat.Ham(req.n, x, z, c)
-        return plan, ham
+        return plan, todo, ham
+
+    def acquire(self, req: Request):
+        return self.acquire_many([req])[0]
+
+    def acquire_many(self, reqs: List[Request]):
+        """(plan, ham) per request, the pooled plans updated together."""
+        got = [self._take(r) for r in reqs]
+        old = [(p, ops) for p, ops, _ in got if ops is not None]
+        nat.update_plans([p for p, _ in old], [ops for _, ops in old])
+        return [(p, h) for p, _, h in got]
 
     def release(self, req: Request, plan, ham) -> None:
         self.plans[(req.n, req.depth)].append(plan)
@@ -225,7 +236,7 @@ class Cache:
 
 def execute_batch(reqs: List[Request], cache: Cache) -> List[Tuple[float, np.ndarray]]:
     """Energies and gradients of small requests in one launch (current stream)."""
-    got = [cache.acquire(r) for r in reqs]
+    got = cache.acquire_many(reqs)
     try:
         # the launch only reads the initial states: one |0> per size
         zero = {n: nat.new_state(n, 0) for n in {r.n for r in reqs}}
