@@ -766,7 +766,7 @@ static int plan_upload_forward(tqsv_plan* p, hipStream_t st) {
   TQSV_HIP(p->uploaded.wait(st));  // an earlier copy on another stream
   const int rc = plan_upload(&p->dprog, &p->dprog_cap, p->prog, st);
   if (rc) return rc;
-  TQSV_HIP(p->uploaded.record(st));
+  p->uploaded.queued(st);
   return 0;
 }
 
@@ -966,7 +966,7 @@ static int plan_upload_adjoint(tqsv_plan* p, hipStream_t st) {
     if (rc) return rc;
     p->uslots = p->hslots;
   }
-  TQSV_HIP(p->uploaded.record(st));
+  p->uploaded.queued(st);
   // the energy partials of a queued H|psi> may already be in the buffer
   const uint32_t eg = ham_apply_grid(p->nu);
   rc = grow_keep(&p->dpartials, &p->dpartials_cap, p->need_partials, 2 * (size_t)eg, st);
@@ -1167,7 +1167,7 @@ int tqsv_ham_set_coeffs(tqsv_ham* h, int nterms, const double* coeff, void* stre
     if (!rc) rc = stage_copy(h->d_stab, tab.data(), tab.size() * sizeof(float2), st);
     if (!rc && !h->diag_terms.empty()) rc = build_diag(h, st);
     if (rc) return rc;
-    TQSV_HIP(h->uploaded.record(st));
+    h->uploaded.queued(st);
     return 0;
   } catch (const std::bad_alloc&) {
     return fail(TQSV_ENOMEM, "tqsv_ham_set_coeffs: out of host memory");

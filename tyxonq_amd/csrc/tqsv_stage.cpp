@@ -5,8 +5,8 @@
 // forward sweep (48 small requests: 256 copies and about 200 waits).
 #include "tqsv_stage.h"
 
+#include <algorithm>
 #include <cstring>
-#include <deque>
 #include <vector>
 
 #include "../../include/tqsv.h"
@@ -16,43 +16,35 @@ namespace tqsv {
 
 namespace {
 
+// The ring is used quarter by quarter.  Before a quarter is written again, the
+// streams of its copies, three quarters ago, are waited for; no event is
+// recorded per copy (an event costs the device about as much as a small copy).
 constexpr size_t kRing = 1 << 20;        // bytes per thread, until the thread ends
-constexpr size_t kLargest = kRing / 4;   // larger copies go from the caller's memory
+constexpr size_t kQuarter = kRing / 4;   // larger copies go from the caller's memory
 
 struct Ring {
-  struct Piece {
-    size_t at, len;
-    hipEvent_t ev;
-  };
   unsigned char* base = nullptr;
   size_t head = 0;
   int dev = -1;
-  std::deque<Piece> busy;  // in ring order, oldest first
-  std::vector<hipEvent_t> idle;
+  std::vector<hipStream_t> users[4];
 
+  hipError_t reclaim(int q) {
+    for (hipStream_t st : users[q])
+      if (hipStreamSynchronize(st) != hipSuccess) {
+        // that stream is gone
+        const hipError_t e = hipDeviceSynchronize();
+        if (e != hipSuccess) return e;
+      }
+    users[q].clear();
+    return hipSuccess;
+  }
   void drop() {
-    for (Piece& p : busy) {
-      (void)hipEventSynchronize(p.ev);
-      (void)hipEventDestroy(p.ev);
-    }
-    for (hipEvent_t e : idle) (void)hipEventDestroy(e);
+    for (int q = 0; q < 4; ++q) (void)reclaim(q);
     if (base) (void)hipHostFree(base);
-    busy.clear();
-    idle.clear();
     base = nullptr;
     head = 0;
   }
   ~Ring() { drop(); }
-
-  // the oldest copy has been made: its memory is free
-  hipError_t retire() {
-    const Piece p = busy.front();
-    const hipError_t e = hipEventSynchronize(p.ev);
-    if (e != hipSuccess) return e;
-    idle.push_back(p.ev);
-    busy.pop_front();
-    return hipSuccess;
-  }
 };
 thread_local Ring g_ring;
 
@@ -64,7 +56,7 @@ int stage_copy(void* dst, const void* src, size_t bytes, hipStream_t st) {
   TQSV_HIP(hipStreamIsCapturing(st, &cs));
   if (cs != hipStreamCaptureStatusNone)
     return fail(TQSV_EUNSUPPORTED, "parameters cannot be replaced under stream capture");
-  if (bytes > kLargest) {
+  if (bytes > kQuarter) {
     TQSV_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
     TQSV_HIP(hipStreamSynchronize(st));
     return 0;
@@ -78,35 +70,16 @@ int stage_copy(void* dst, const void* src, size_t bytes, hipStream_t st) {
     r.dev = dev;
   }
   const size_t len = (bytes + 63) & ~(size_t)63;
-  // pieces are taken in ring order, so those in the way are the oldest (at a
-  // wrap, first those between the head and the end)
-  if (r.head + len > kRing) {
-    while (!r.busy.empty() && r.busy.front().at >= r.head) TQSV_HIP(r.retire());
-    r.head = 0;
-  }
-  const size_t at = r.head;
-  while (!r.busy.empty() && r.busy.front().at < at + len && at < r.busy.front().at + r.busy.front().len)
-    TQSV_HIP(r.retire());
-  if (r.busy.size() >= 256) TQSV_HIP(r.retire());  // bounded number of events
-  hipEvent_t ev = nullptr;
-  if (!r.idle.empty()) {
-    ev = r.idle.back();
-    r.idle.pop_back();
-  } else {
-    TQSV_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-  }
-  std::memcpy(r.base + at, src, bytes);
-  hipError_t e = hipMemcpyAsync(dst, r.base + at, bytes, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) {
-    e = hipEventRecord(ev, st);
-    if (e != hipSuccess) (void)hipStreamSynchronize(st);
-  }
-  if (e != hipSuccess) {
-    (void)hipEventDestroy(ev);
-    return hip_fail(e, "stage_copy");
-  }
-  r.busy.push_back(Ring::Piece{at, len, ev});
-  r.head = at + len;
+  // a copy lies within one quarter
+  if (r.head % kQuarter + len > kQuarter || r.head == kRing)
+    r.head = (r.head + kQuarter - 1) / kQuarter * kQuarter % kRing;
+  const int q = (int)(r.head / kQuarter);
+  if (r.head % kQuarter == 0) TQSV_HIP(r.reclaim(q));
+  std::memcpy(r.base + r.head, src, bytes);
+  TQSV_HIP(hipMemcpyAsync(dst, r.base + r.head, bytes, hipMemcpyHostToDevice, st));
+  if (std::find(r.users[q].begin(), r.users[q].end(), st) == r.users[q].end())
+    r.users[q].push_back(st);
+  r.head += len;
   return 0;
 }
 

@@ -13,8 +13,9 @@ namespace tqsv {
 // copies left in the staging buffer.
 int stage_copy(void* dst, const void* src, size_t bytes, hipStream_t st);
 
-// What was queued for an object on one stream, to be waited for by uses on
-// another (uses on the same stream follow it anyway).
+// The stream on which copies for an object were queued.  Uses on that stream
+// follow them anyway; a use on another stream waits for it, through an event
+// that is recorded at the first such use (a record is a packet for the device to process).
 class StreamMark {
  public:
   StreamMark() = default;
@@ -23,24 +24,28 @@ class StreamMark {
   ~StreamMark() {
     if (ev_) (void)hipEventDestroy(ev_);
   }
-  hipError_t record(hipStream_t st) {
-    if (!ev_) {
-      const hipError_t e = hipEventCreateWithFlags(&ev_, hipEventDisableTiming);
-      if (e != hipSuccess) return e;
-    }
+  void queued(hipStream_t st) {
     st_ = st;
     set_ = true;
-    return hipEventRecord(ev_, st);
+    recorded_ = false;
   }
   void clear() { set_ = false; }
-  // a stream under capture cannot wait for work outside the capture: the host
-  // waits, once
   hipError_t wait(hipStream_t st) {
     if (!set_ || st == st_) return hipSuccess;
+    hipError_t e = ev_ ? hipSuccess : hipEventCreateWithFlags(&ev_, hipEventDisableTiming);
+    if (e != hipSuccess) return e;
+    if (!recorded_ && hipEventRecord(ev_, st_) != hipSuccess) {
+      // that stream is gone
+      clear();
+      return hipDeviceSynchronize();
+    }
+    recorded_ = true;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    hipError_t e = hipStreamIsCapturing(st, &cs);
+    e = hipStreamIsCapturing(st, &cs);
     if (e != hipSuccess) return e;
     if (cs == hipStreamCaptureStatusNone) return hipStreamWaitEvent(st, ev_, 0);
+    // a stream under capture cannot wait for work outside the capture: the
+    // host waits, once
     e = hipEventSynchronize(ev_);
     if (e == hipSuccess) clear();
     return e;
@@ -49,7 +54,7 @@ class StreamMark {
  private:
   hipEvent_t ev_ = nullptr;
   hipStream_t st_ = nullptr;
-  bool set_ = false;
+  bool set_ = false, recorded_ = false;
 };
 
 }  // namespace tqsv
