@@ -16,9 +16,9 @@
 // per chunk of 64 columns of U for k >= 7, where each work-group computes 64
 // of the 2^k output rows.
 // Measured per call (one thread per amplitude -> here; random targets): 24
-// qubits, k = 3: 178 -> 72-86 us, 4: 379 -> 60, 5: 704 -> 83, 6: 1017 -> 116 (the
-// kernel about 90: 95 TFLOP/s of the 150 a large FP32 matrix product reaches);
-// 27 qubits, k = 5: 4.41 -> 0.50 ms (4.3 TB/s); 24 qubits, k = 8: 8.9 -> 0.46 ms.
+// qubits, k = 3: 178 -> 72 us, 4: 379 -> 58, 5: 704 -> 72, 6: 1017 -> 114 (75
+// TFLOP/s with the call, of the 150 a large FP32 matrix product reaches); 27
+// qubits, k = 5: 4.41 -> 0.45 ms (4.8 TB/s); 24 qubits, k = 8: 8.9 -> 0.35 ms.
 // Error against 64 bits at k = 6: 1.5e-7 -> 1.1e-7.
 #include <hip/hip_runtime.h>
 
@@ -67,7 +67,7 @@ __host__ __device__ constexpr uint32_t rev5(uint32_t r) {
 }
 
 template <int LK, bool MULTI>
-__global__ __launch_bounds__(256) void kq_mfma_kernel(const float2* __restrict__ psi,
+__global__ __launch_bounds__(256, 2) void kq_mfma_kernel(const float2* __restrict__ psi,
                                                       float2* __restrict__ out, KqGeo g,
                                                       const float2* __restrict__ A,
                                                       uint32_t nwork) {
@@ -231,8 +231,11 @@ hipError_t k_apply_kq_mfma(const float2* psi, float2* out, int k, const KqGeo& g
                            hipStream_t st) {
   const uint64_t nwork = (uint64_t)g.ntiles * g.nchunk;
   if (nwork > 0xffffffffull - 4096u) return hipErrorInvalidValue;
-  // 3 work-groups per CU fit by registers and LDS; each loops over its tiles
-  const uint32_t grid = (uint32_t)(nwork < 768u ? nwork : 768u);
+  // 2 work-groups per CU fit by registers; 4 to 8 tiles each balance the load
+  // (24 qubits, k = 5: 512 or 1024 work-groups 71 us, 768 82; 27 qubits, k = 5:
+  // 1024 516 us, 4096 449)
+  const uint64_t want = nwork / 8 < 1024u ? 1024u : (nwork / 8 > 4096u ? 4096u : nwork / 8);
+  const uint32_t grid = (uint32_t)(nwork < want ? nwork : want);
   const dim3 G(grid), B(256);
   const uint32_t nw = (uint32_t)nwork;
   if (k == 4)
