@@ -13,6 +13,9 @@
 // equal) on the CUs that have a tile.  Measured per pass, 2^13-amplitude tiles,
 // 18 qubits (32 tiles), about 50 gates: gate 75 -> 34 us, dual 287 -> 108 us;
 // 14 qubits (2 tiles), UCCSD rotation groups: gate 211 -> 127, dual 454 -> 329 us.
+// With 2^12 tiles, and the register positions' index bits and LDS offsets from
+// the phase header (one load) instead of formed per phase: 18 qubits gate 19.8
+// -> 18.6, dual 45.3 -> 35.4 us; 14 qubits gate 34.4 -> 30.0, dual 76 -> 64 us.
 #ifndef TQSV_INTERP_H
 #define TQSV_INTERP_H
 
@@ -24,19 +27,6 @@
 namespace tqsv {
 
 constexpr int NR = NSLOT / 4;  // slots per lane
-
-// LDS position of a tile position: linear over GF(2); bit 0 is preserved, so
-// pairs stay 16-byte aligned.  Bits 5-13 are spread over the bank bits so that a
-// phase's reads (two register positions and the lowest free positions across
-// the lanes) meet few conflicts wherever the register positions lie.
-__device__ __forceinline__ uint32_t swq(uint32_t p) {
-  const uint32_t t = p >> 5;
-  const uint32_t e4 = (t ^ (t >> 2) ^ (t >> 4) ^ (t >> 6) ^ (t >> 8)) & 1u;
-  const uint32_t e3 = ((t >> 1) ^ (t >> 3) ^ (t >> 5) ^ (t >> 7)) & 1u;
-  const uint32_t e2 = ((t >> 2) ^ (t >> 6)) & 1u;
-  const uint32_t e1 = ((t >> 3) ^ (t >> 7)) & 1u;
-  return p ^ (e4 << 4) ^ (e3 << 3) ^ (e2 << 2) ^ (e1 << 1);
-}
 
 // first words of a step; the next step's are fetched while one runs (programs
 // on the device are followed by STEP_SLACK words)
@@ -376,6 +366,8 @@ __device__ __forceinline__ void put_red(float v, double* acc, uint32_t nred, uin
   if ((threadIdx.x & 63u) == 63u) acc[(threadIdx.x >> 6) * nred + slot] += d;
 }
 
+// Runs the step h at w.  (Nothing here may depend on the next step's words: they
+// would be waited for before this step's work.)
 template <int MODE, typename IDX>
 __device__ __forceinline__ void run_step(const step_t& h, cw_t w, float2 (&a)[NR], float2 (&b)[NR],
                                          QuadGeo<IDX> G, double* acc, uint32_t nred) {
@@ -542,49 +534,55 @@ __device__ __forceinline__ void run_step(const step_t& h, cw_t w, float2 (&a)[NR
       }
       break;
     }
-    case OP_PROT:
+    case OP_PROT: {
+      float2 p[NR];
+      const IDX z = widx<IDX>(h[2], h[3]);
+      const uint32_t xr = h[1], k = (h[6] + 3u) & 3u;  // -i i^|x&z| = i^k
+      // the partner's sign; i^(k + 2) = -i^k
+      uint32_t ts = (uint32_t)(parity((IDX)((G.gb ^ G.gq) & z)) ^ (h[6] & 1u)) << 31;
+      if (xr != 0) ts ^= (k & 2u) << 30;
+      uint32_t sm = 0;
+#pragma unroll
+      for (int s = 0; s < NR; ++s) sm |= (uint32_t)parity((IDX)(gs_reg(G, s) & z)) << s;
+      partner(xr, a, p);
+      qprot(a, p, xr == 0, F(4), F(5), k & 1u, ts, sm);
+      if constexpr (DUAL) {
+        partner(xr, b, p);
+        qprot(b, p, xr == 0, F(4), F(5), k & 1u, ts, sm);
+      }
+      break;
+    }
     case OP_PGRP: {
       float2 p[NR];
-      auto both = [&](auto&& f) {
-        partner(h[1], a, p);
-        f(a);
-        if constexpr (DUAL) {
-          partner(h[1], b, p);
-          f(b);
+      const uint32_t xr = h[1], sm = h[6];
+      const uint32_t ts =
+          (uint32_t)(parity((IDX)(G.gb & widx<IDX>(h[2], h[3]))) ^ ((sm >> q) & 1u) ^ (h[4] & 1u)) << 31;
+      uint32_t Mi = 0, Mj = 0;
+      partner(xr, a, p);
+      for (uint32_t act = h[5]; act; act &= act - 1u) {
+        const uint32_t c = (uint32_t)__builtin_ctz(act);
+        class_slots(xr, c, Mi, Mj);
+        qpgrp(a, p, Mi, Mj, q, w + PG_HDR + PG_ENT * c, ts, sm);
+      }
+      if constexpr (DUAL) {
+        partner(xr, b, p);
+        const bool one = (h[5] & (h[5] - 1u)) == 0;  // the masks are still its
+        for (uint32_t act = h[5]; act; act &= act - 1u) {
+          const uint32_t c = (uint32_t)__builtin_ctz(act);
+          if (!one) class_slots(xr, c, Mi, Mj);
+          qpgrp(b, p, Mi, Mj, q, w + PG_HDR + PG_ENT * c, ts, sm);
         }
-      };
-      const IDX z = widx<IDX>(h[2], h[3]);
-      if ((h[0] & 0xffffu) == OP_PROT) {
-        const uint32_t xr = h[1], k = (h[6] + 3u) & 3u;  // -i i^|x&z| = i^k
-        // the partner's sign; i^(k + 2) = -i^k
-        uint32_t ts = (uint32_t)(parity((IDX)((G.gb ^ G.gq) & z)) ^ (h[6] & 1u)) << 31;
-        if (xr != 0) ts ^= (k & 2u) << 30;
-        uint32_t sm = 0;
-#pragma unroll
-        for (int s = 0; s < NR; ++s) sm |= (uint32_t)parity((IDX)(gs_reg(G, s) & z)) << s;
-        both([&](float2 (&v)[NR]) { qprot(v, p, xr == 0, F(4), F(5), k & 1u, ts, sm); });
-      } else {
-        const uint32_t xr = h[1], sm = h[6];
-        const uint32_t ts = (uint32_t)(parity((IDX)(G.gb & z)) ^ ((sm >> q) & 1u) ^ (h[4] & 1u)) << 31;
-        both([&](float2 (&v)[NR]) {
-          for (uint32_t act = h[5]; act; act &= act - 1u) {
-            const uint32_t c = (uint32_t)__builtin_ctz(act);
-            uint32_t Mi, Mj;
-            class_slots(xr, c, Mi, Mj);
-            qpgrp(v, p, Mi, Mj, q, w + PG_HDR + PG_ENT * c, ts, sm);
-          }
-        });
       }
       break;
     }
     case OP_RED: {
       if constexpr (DUAL) {
         const uint32_t xr = h[1], slot = h[4], sm = h[7];
+        // slot signs are a parity of the slot bits: the lane's part once
         const uint32_t tp = parity((IDX)(G.gb & widx<IDX>(h[5], h[6]))) ^ ((sm >> q) & 1u);
         float2 p[NR];
         partner(xr, a, p);
         if (h[2] == RED_CROSS) {
-          // slot signs are a parity of the slot bits: the lane's part once
           float v0 = 0.f, v1 = 0.f;
           if (h[8]) {
 #pragma unroll
@@ -645,7 +643,8 @@ __device__ __forceinline__ void run_phases(cw_t prog, float2* tA, float2* tB, do
   const uint32_t nphase = prog[PH_NPHASE];
   cw_t ph = prog + PH_SIZE;
   for (uint32_t iph = 0; iph < nphase; ++iph) {
-    const uint32_t nsteps = ph[PS_NSTEPS];
+    const step_t hd = *(cstep_t)ph;  // (PS_SIZE words)
+    const uint32_t nsteps = hd[PS_NSTEPS];
     cw_t w = ph + PS_SIZE;
 #pragma unroll 1
     for (int turn = 0; turn < TURNS; ++turn) {
@@ -656,10 +655,10 @@ __device__ __forceinline__ void run_phases(cw_t prog, float2* tA, float2* tB, do
       G.rmask = 0;
 #pragma unroll
       for (int j = 0; j < RB; ++j) {
-        const uint32_t r = ph[PS_R + j];
+        const uint32_t r = hd[PS_R + j];
         tpos = ((tpos >> r) << (r + 1)) | (tpos & ((1u << r) - 1u));
-        sp[j] = swq(1u << r);
-        gR[j] = (IDX)1 << (r < tb.L ? r : prog[PH_H + (r < tb.L ? 0u : r - tb.L)]);
+        sp[j] = hd[PS_S + j];
+        gR[j] = (IDX)1 << hd[PS_G + j];
         G.rmask |= gR[j];
       }
       G.q = q;

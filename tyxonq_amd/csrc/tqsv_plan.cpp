@@ -1409,7 +1409,12 @@ int emit_passes(std::vector<Gate>& gates, const SchedOpts& so, std::vector<PassP
       uint32_t nsteps = 0;
       for (size_t at = steps0; at < prog.size(); at += prog[at] >> 16) ++nsteps;
       prog[hdr + PS_NSTEPS] = nsteps;
-      for (int r = 0; r < RB; ++r) prog[hdr + PS_R + r] = pp.Rpos[ip][r];
+      for (int r = 0; r < RB; ++r) {
+        const uint32_t R = pp.Rpos[ip][r];
+        prog[hdr + PS_R + r] = R;
+        prog[hdr + PS_G + r] = R < pp.L ? R : pp.H[R - pp.L];
+        prog[hdr + PS_S + r] = swq(1u << R);
+      }
     }
     uint32_t* h = prog.data() + pp.prog_off;
     h[PH_FLAGS] = PF_WRITE | (so.dual ? PF_DUAL : 0u);

@@ -50,7 +50,25 @@ constexpr int PH_SIZE = PH_H + MAXH + 3;  // 20 words
 // phase header
 constexpr int PS_NSTEPS = 0;
 constexpr int PS_R = 1;           // R[0..RB), ascending
-constexpr int PS_SIZE = 8;
+// gate and dual passes, for the interpreting kernel: the global index bit and
+// the LDS offset (swq) of each register position
+constexpr int PS_G = 6;
+constexpr int PS_S = 11;
+constexpr int PS_SIZE = 16;
+
+// LDS position of a tile position in the interpreting kernel: linear over
+// GF(2); bit 0 is preserved, so pairs stay 16-byte aligned.  Bits 5-13 are spread
+// over the bank bits so that a phase's reads (two register positions and the
+// lowest free positions across the lanes) meet few conflicts wherever the
+// register positions lie.
+constexpr uint32_t swq(uint32_t p) {
+  const uint32_t t = p >> 5;
+  const uint32_t e4 = (t ^ (t >> 2) ^ (t >> 4) ^ (t >> 6) ^ (t >> 8)) & 1u;
+  const uint32_t e3 = ((t >> 1) ^ (t >> 3) ^ (t >> 5) ^ (t >> 7)) & 1u;
+  const uint32_t e2 = ((t >> 2) ^ (t >> 6)) & 1u;
+  const uint32_t e1 = ((t >> 3) ^ (t >> 7)) & 1u;
+  return p ^ (e4 << 4) ^ (e3 << 3) ^ (e2 << 2) ^ (e1 << 1);
+}
 
 // Step word 0: opcode | (nwords << 16); all offsets below are from the step
 // start.  "k" is a slot bit (0..RB-1); "g" is a global index bit.
