@@ -216,6 +216,10 @@ def _ptr(t) -> int:
         raise TypeError("expected a complex64 tensor on the GPU")
     if not t.is_contiguous():
         raise ValueError("state tensor must be contiguous")
+    if t.is_conj() or t.is_neg():
+        # the memory holds the values before the conjugation or sign change
+        raise ValueError("state tensor is a lazy conjugate or negation: pass resolve_conj() / "
+                         "resolve_neg() of it")
     return int(t.data_ptr())
 
 
@@ -332,6 +336,8 @@ def z_grad(psi, bit: int, ge):
     torch = _torch()
     if ge.dtype != torch.float64 or not ge.is_cuda or ge.numel() != 1:
         raise TypeError("expected one float64 on the GPU")
+    if ge.is_neg():
+        raise ValueError("the factor is a lazy negation: pass resolve_neg() of it")
     out = torch.empty_like(psi)
     _check(load().tqsv_z_grad(_ptr(psi), _ptr(out), _nqubits(psi), int(bit), ge.data_ptr(),
                               stream_ptr()))

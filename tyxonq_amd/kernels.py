@@ -54,7 +54,13 @@ def _as_state(state: Any, num_qubits: int):
                                                              dtype=torch.complex64)
     if t.numel() != (1 << int(num_qubits)):
         raise ValueError(f"state has {t.numel()} amplitudes, expected 2^{num_qubits}")
-    return t.contiguous()
+    return _resolved(t.contiguous())
+
+
+def _resolved(t: Any):
+    """t with a pending conjugation or sign change written out: the kernels read
+    the memory, and reshape, contiguous and .to() keep those flags."""
+    return t.resolve_conj().resolve_neg()
 
 
 def _mat(m: Any, dim: int) -> np.ndarray:
@@ -104,8 +110,8 @@ def _apply_function():
 
         @staticmethod
         def backward(ctx, gout):
-            g = gout.detach().to(device=nat.device(), dtype=torch.complex64).reshape(-1) \
-                .contiguous()
+            g = _resolved(gout.detach().to(device=nat.device(), dtype=torch.complex64)
+                          .reshape(-1).contiguous())
             gs = gU = None
             if ctx.needs_input_grad[0]:
                 gs = _apply_new(g, ctx.bits, ctx.U.conj().T)
@@ -141,7 +147,7 @@ def _expect_z_function():
         @staticmethod
         def backward(ctx, ge):
             (psi,) = ctx.saved_tensors
-            g = ge.detach().to(device=psi.device, dtype=torch.float64)
+            g = _resolved(ge.detach().to(device=psi.device, dtype=torch.float64))
             zpsi = nat.z_grad(psi, ctx.bit, g)
             dt, dev, shape = ctx.state_meta
             return zpsi.to(device=dev, dtype=dt if dt.is_complex else torch.complex128) \
@@ -170,6 +176,11 @@ def _inplace_state(state: Any, num_qubits: int):
     if _tracked(state):
         raise ValueError("in-place kernels cannot take a state that requires grad; "
                          "use the out-of-place function")
+    # (other types and devices are converted, and with that written out, anyway)
+    if getattr(state, "is_cuda", False) and state.dtype == _torch().complex64 and \
+            (state.is_conj() or state.is_neg()):
+        raise ValueError("in-place kernels cannot take a lazily conjugated or negated state; "
+                         "use the out-of-place function or resolve_conj()")
     return _as_state(state, num_qubits)
 
 
