@@ -1162,13 +1162,13 @@ int tqsv_ham_set_coeffs(tqsv_ham* h, int nterms, const double* coeff, void* stre
     const std::vector<float2> tab = sub_tables(h);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     TQSV_HIP(h->uploaded.wait(st));
-    int rc = stage_copy(h->d_tc, tc.data(), tc.size() * sizeof(float2), st);
+    // the diagonal's kernel first: the place of the last copy is also after it
+    int rc = h->diag_terms.empty() ? 0 : build_diag(h, st);
     if (!rc) rc = stage_copy(h->d_rtc, rtc.data(), rtc.size() * sizeof(float2), st);
     if (!rc) rc = stage_copy(h->d_stab, tab.data(), tab.size() * sizeof(float2), st);
-    if (!rc && !h->diag_terms.empty()) rc = build_diag(h, st);
-    if (rc) return rc;
+    if (!rc) rc = stage_copy(h->d_tc, tc.data(), tc.size() * sizeof(float2), st);
     h->uploaded.queued(st);
-    return 0;
+    return rc;
   } catch (const std::bad_alloc&) {
     return fail(TQSV_ENOMEM, "tqsv_ham_set_coeffs: out of host memory");
   }

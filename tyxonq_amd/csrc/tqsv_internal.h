@@ -57,6 +57,13 @@ hipError_t k_project_zero(float2* psi, int n, int bit, int keep, hipStream_t st)
 hipError_t k_scale(float2* psi, int n, float re, float im, hipStream_t st);
 // dst[i] = i < nsrc ? src[i] : 0 for i < ndst (src may be NULL when nsrc = 0)
 hipError_t k_pad_copy(const float2* src, uint64_t nsrc, float2* dst, uint64_t ndst, hipStream_t st);
+// Copies whole 4-byte words from page-locked host memory in pieces of STAGE_PIECE
+// bytes; piece p, when it is done, writes number + p to word (number + p) % nwords
+// (page-locked host memory).
+constexpr size_t STAGE_PIECE = 4096;
+inline uint32_t stage_pieces(size_t bytes) { return (uint32_t)((bytes + STAGE_PIECE - 1) / STAGE_PIECE); }
+hipError_t k_stage_copy(void* dst, const void* src, size_t bytes, uint64_t* words, uint64_t nwords,
+                        uint64_t number, hipStream_t st);
 hipError_t k_apply_kq(const float2* psi, float2* out, int n, int k, const uint32_t* bitpos,
                       const uint64_t* off, const float2* U, hipStream_t st);
 // Matrix-core form of the same (tqsv_kq.hip): tiles of 2^KQ_TILE_BITS

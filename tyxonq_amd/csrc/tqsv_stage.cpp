@@ -5,44 +5,90 @@
 // forward sweep (48 small requests: 256 copies and about 200 waits).
 #include "tqsv_stage.h"
 
-#include <algorithm>
+#include <atomic>
 #include <cstring>
-#include <vector>
+#include <thread>
 
 #include "../../include/tqsv.h"
 #include "tqsv_internal.h"
 
 namespace tqsv {
 
+// The pieces (k_stage_copy) of a thread's copies are numbered.  A piece that has
+// run writes its number to word (number % kWords) of page-locked memory; a word is
+// used again only when its last number is there.  So "has this copy run" is a
+// read of host memory, whatever has become of the copy's stream since.
+struct StageTickets {
+  static constexpr uint64_t kWords = 2048;
+  std::mutex m;
+  uint64_t* word = nullptr;  // NULL: every copy has run and the thread is done with it
+
+  bool reached(uint64_t t) {
+    std::lock_guard<std::mutex> lock(m);
+    return !word || __atomic_load_n(&word[t % kWords], __ATOMIC_ACQUIRE) >= t;
+  }
+  void wait(uint64_t first, uint64_t last) {
+    for (uint64_t t = first; t <= last; ++t)
+      for (int k = 0; !reached(t); ++k)
+        if (k >= 64) std::this_thread::yield();
+  }
+};
+
+void StagePoint::wait() const {
+  if (of) of->wait(first, last);
+}
+
 namespace {
 
-// The ring is used quarter by quarter.  Before a quarter is written again, the
-// streams of its copies, three quarters ago, are waited for; no event is
-// recorded per copy (an event costs the device about as much as a small copy).
+// The ring is used quarter by quarter; before a quarter is written again, its
+// copies, three quarters ago, are waited for.
 constexpr size_t kRing = 1 << 20;        // bytes per thread, until the thread ends
 constexpr size_t kQuarter = kRing / 4;   // larger copies go from the caller's memory
 
 struct Ring {
-  unsigned char* base = nullptr;
+  unsigned char* base = nullptr;  // the ring, then the words of the tickets
   size_t head = 0;
   int dev = -1;
-  std::vector<hipStream_t> users[4];
+  std::shared_ptr<StageTickets> tickets;
+  uint64_t next = 1;              // numbers start at 1: a word of 0 holds none
+  uint64_t latest = 0;            // first number of the last copy
+  struct {
+    uint64_t first = 1, last = 0;
+  } quarter[4];                   // numbers of each quarter's copies
 
-  hipError_t reclaim(int q) {
-    for (hipStream_t st : users[q])
-      if (hipStreamSynchronize(st) != hipSuccess) {
-        // that stream is gone
-        const hipError_t e = hipDeviceSynchronize();
-        if (e != hipSuccess) return e;
-      }
-    users[q].clear();
-    return hipSuccess;
+  int open(int device) {
+    drop();
+    const size_t words = StageTickets::kWords * sizeof(uint64_t);
+    auto t = std::make_shared<StageTickets>();
+    // (another thread may be capturing: an allocation is no part of that)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    TQSV_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&base), kRing + words,
+                                       hipHostMallocCoherent | hipHostMallocPortable);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+      base = nullptr;
+      return hip_fail(e, "staging ring");
+    }
+    t->word = reinterpret_cast<uint64_t*>(base + kRing);
+    std::memset(t->word, 0, words);
+    tickets = std::move(t);
+    dev = device;
+    return 0;
   }
   void drop() {
-    for (int q = 0; q < 4; ++q) (void)reclaim(q);
-    if (base) (void)hipHostFree(base);
+    if (!base) return;
+    tickets->wait(next > StageTickets::kWords ? next - StageTickets::kWords : 1, next - 1);
+    {
+      std::lock_guard<std::mutex> lock(tickets->m);
+      tickets->word = nullptr;
+    }
+    (void)hipHostFree(base);
     base = nullptr;
+    tickets.reset();
     head = 0;
+    next = 1;
+    for (auto& q : quarter) q = {};
   }
   ~Ring() { drop(); }
 };
@@ -50,13 +96,18 @@ thread_local Ring g_ring;
 
 }  // namespace
 
+StagePoint stage_point() {
+  const Ring& r = g_ring;
+  return r.base ? StagePoint{r.tickets, r.latest, r.next - 1} : StagePoint{};
+}
+
 int stage_copy(void* dst, const void* src, size_t bytes, hipStream_t st) {
   if (bytes == 0) return 0;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   TQSV_HIP(hipStreamIsCapturing(st, &cs));
   if (cs != hipStreamCaptureStatusNone)
     return fail(TQSV_EUNSUPPORTED, "parameters cannot be replaced under stream capture");
-  if (bytes > kQuarter) {
+  if (bytes > kQuarter || bytes % 4 != 0) {
     TQSV_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
     TQSV_HIP(hipStreamSynchronize(st));
     return 0;
@@ -65,20 +116,29 @@ int stage_copy(void* dst, const void* src, size_t bytes, hipStream_t st) {
   int dev = 0;
   TQSV_HIP(hipGetDevice(&dev));
   if (!r.base || r.dev != dev) {
-    r.drop();
-    TQSV_HIP(hipHostMalloc(reinterpret_cast<void**>(&r.base), kRing, hipHostMallocDefault));
-    r.dev = dev;
+    const int rc = r.open(dev);
+    if (rc) return rc;
   }
   const size_t len = (bytes + 63) & ~(size_t)63;
   // a copy lies within one quarter
   if (r.head % kQuarter + len > kQuarter || r.head == kRing)
     r.head = (r.head + kQuarter - 1) / kQuarter * kQuarter % kRing;
-  const int q = (int)(r.head / kQuarter);
-  if (r.head % kQuarter == 0) TQSV_HIP(r.reclaim(q));
+  auto& q = r.quarter[r.head / kQuarter];
+  if (r.head % kQuarter == 0) {
+    r.tickets->wait(q.first, q.last);
+    q.last = 0;
+  }
+  const uint64_t t = r.next, end = t + stage_pieces(bytes);
+  // the words of these numbers
+  if (end > StageTickets::kWords + 1)
+    r.tickets->wait(t > StageTickets::kWords ? t - StageTickets::kWords : 1,
+                    end - 1 - StageTickets::kWords);
   std::memcpy(r.base + r.head, src, bytes);
-  TQSV_HIP(hipMemcpyAsync(dst, r.base + r.head, bytes, hipMemcpyHostToDevice, st));
-  if (std::find(r.users[q].begin(), r.users[q].end(), st) == r.users[q].end())
-    r.users[q].push_back(st);
+  TQSV_HIP(k_stage_copy(dst, r.base + r.head, bytes, r.tickets->word, StageTickets::kWords, t, st));
+  if (!q.last) q.first = t;
+  q.last = end - 1;
+  r.latest = t;
+  r.next = end;
   r.head += len;
   return 0;
 }

@@ -5,56 +5,64 @@
 
 #include <hip/hip_runtime.h>
 #include <stddef.h>
+#include <stdint.h>
+
+#include <memory>
+#include <mutex>
 
 namespace tqsv {
+
+struct StageTickets;
+
+// A place in a thread's sequence of staged copies: reached when the pieces with
+// these numbers, and with them what their stream held before, have run.
+struct StagePoint {
+  std::shared_ptr<StageTickets> of;
+  uint64_t first = 0, last = 0;
+  // the host waits; no call on any stream
+  void wait() const;
+};
 
 // Queues the copy of `bytes` from host memory (free to change or go on return)
 // to the device.  Refused under stream capture: a replay would read what later
 // copies left in the staging buffer.
 int stage_copy(void* dst, const void* src, size_t bytes, hipStream_t st);
+// the calling thread's last staged copy
+StagePoint stage_point();
 
-// The stream on which copies for an object were queued.  Uses on that stream
-// follow them anyway; a use on another stream waits for it, through an event
-// that is recorded at the first such use (a record is a packet for the device to process).
+// The stream on which copies for an object were queued, and their place.  Uses
+// on that stream follow them anyway; the first use on another one waits on the
+// host until they have run (a device-side wait needs an event, which is a
+// packet for the device at every update, or recorded later on a stream that
+// may be under capture, or gone, by then).  Several threads may use an object.
 class StreamMark {
  public:
   StreamMark() = default;
   StreamMark(const StreamMark&) = delete;
   StreamMark& operator=(const StreamMark&) = delete;
-  ~StreamMark() {
-    if (ev_) (void)hipEventDestroy(ev_);
-  }
+  // the calling thread's staged copies so far
   void queued(hipStream_t st) {
+    std::lock_guard<std::mutex> lock(m_);
+    at_ = stage_point();
     st_ = st;
-    set_ = true;
-    recorded_ = false;
   }
-  void clear() { set_ = false; }
+  void clear() {
+    std::lock_guard<std::mutex> lock(m_);
+    at_ = StagePoint{};
+  }
   hipError_t wait(hipStream_t st) {
-    if (!set_ || st == st_) return hipSuccess;
-    hipError_t e = ev_ ? hipSuccess : hipEventCreateWithFlags(&ev_, hipEventDisableTiming);
-    if (e != hipSuccess) return e;
-    if (!recorded_ && hipEventRecord(ev_, st_) != hipSuccess) {
-      // that stream is gone
-      clear();
-      return hipDeviceSynchronize();
-    }
-    recorded_ = true;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    e = hipStreamIsCapturing(st, &cs);
-    if (e != hipSuccess) return e;
-    if (cs == hipStreamCaptureStatusNone) return hipStreamWaitEvent(st, ev_, 0);
-    // a stream under capture cannot wait for work outside the capture: the
-    // host waits, once
-    e = hipEventSynchronize(ev_);
-    if (e == hipSuccess) clear();
-    return e;
+    std::lock_guard<std::mutex> lock(m_);
+    // (each thread has a stream of its own behind hipStreamPerThread)
+    if (!at_.of || (st == st_ && st != hipStreamPerThread)) return hipSuccess;
+    at_.wait();
+    at_ = StagePoint{};
+    return hipSuccess;
   }
 
  private:
-  hipEvent_t ev_ = nullptr;
+  std::mutex m_;
+  StagePoint at_;
   hipStream_t st_ = nullptr;
-  bool set_ = false, recorded_ = false;
 };
 
 }  // namespace tqsv
