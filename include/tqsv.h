@@ -228,7 +228,10 @@ int tqsv_plan_create(int n, const tqsv_op* ops, int nops, const tqsv_plan_opts* 
                      tqsv_plan** out);
 
 /* Replace the parameters (matrices, angles) of a plan whose op structure is
- * unchanged (same kinds, targets, controls, masks) and re-upload. */
+ * unchanged (same kinds, targets, controls, masks) and re-upload.  The copies are
+ * queued on `stream`; later uses of the plan, on any stream, come after them.  Once
+ * the plan has been used under stream capture, the call returns when the copies
+ * have run, so that replays launched after it read the new parameters. */
 int tqsv_plan_update(tqsv_plan* plan, const tqsv_op* ops, int nops, void* stream);
 
 /* tqsv_plan_update of several plans at once: the programs are written on several
@@ -296,8 +299,8 @@ int tqsv_ham_precompile(int n, int nterms, const uint64_t* xmask, const uint64_t
  * divided by the norm. */
 /* Replace the coefficients of a Hamiltonian (same terms, same order), e.g. a
  * field strength that changes between requests; the term structure and the
- * device plans are kept.  No counterpart in the reference (whose Pauli sums
- * are plain lists, vqe.py:9-20). */
+ * device plans are kept.  Queued and ordered like tqsv_plan_update.  No
+ * counterpart in the reference (whose Pauli sums are plain lists, vqe.py:9-20). */
 int tqsv_ham_set_coeffs(tqsv_ham* ham, int nterms, const double* coeff, void* stream);
 
 int tqsv_ham_expval(tqsv_ham* ham, const void* psi, double* terms, double* energy,

@@ -283,6 +283,41 @@ void updater_under_capture() {
   expect(all(got, 7), "the table was read before its copy");
 }
 
+// updated and captured on one stream: the graph is replayed on another
+void capture_on_own_stream() {
+  Stream a, b;
+  Object o;
+  a.hold(true);
+  o.update(a, 7);
+  a.capturing = true;
+  Release r(a, 50);
+  expect(o.mark.wait(H(a)) == hipSuccess, "wait failed");
+  a.capturing = false;
+  std::vector<uint32_t> got;
+  b.push([&] { got = o.dev; });  // the replay
+  b.drain();
+  expect(all(got, 7), "the replay read the table before its copy");
+}
+
+// an object used under capture is updated, and the graph replayed elsewhere
+void update_after_capture() {
+  Stream a, b;
+  Object o;
+  o.update(a, 7);
+  b.capturing = true;
+  expect(o.mark.wait(H(b)) == hipSuccess, "wait failed");
+  b.capturing = false;
+  for (uint32_t v = 8; v < 11; ++v) {
+    a.hold(true);
+    Release r(a, 30);
+    o.update(a, v);
+    std::vector<uint32_t> got;
+    b.push([&] { got = o.dev; });  // the replay
+    b.drain();
+    expect(all(got, v), "the replay read the table before its copy");
+  }
+}
+
 // the ring comes round while a stream of earlier copies is under capture, or gone
 void ring(bool gone) {
   Stream a, b;
@@ -358,6 +393,8 @@ int main(int argc, char** argv) {
   const std::string w = argc > 1 ? argv[1] : "";
   if (w == "two_threads") two_threads();
   else if (w == "updater_under_capture") updater_under_capture();
+  else if (w == "capture_on_own_stream") capture_on_own_stream();
+  else if (w == "update_after_capture") update_after_capture();
   else if (w == "ring_capture") ring(false);
   else if (w == "ring_gone") ring(true);
   else if (w == "in_flight") in_flight();

@@ -106,6 +106,48 @@ def test_update_used_on_another_stream_and_under_capture(gpu):
             plan.update(_rows(3))
 
 
+def test_updates_between_replays_on_another_stream(gpu):
+    """A replay passes no host call: updates of a captured plan and Hamiltonian
+    are complete when they return."""
+    import torch
+
+    from tyxonq_amd import _native as nat
+
+    plan = nat.Plan(N, _rows(0))
+    ham, nt = _ham(1.0)
+    psi, out = nat.new_state(N, 0), nat.new_state(N, 0)
+
+    def go():
+        nat.init_basis(psi, 0)
+        plan.run(psi)
+        ham.apply(psi, out)
+
+    go()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        go()
+    want = []
+    for k in range(3):
+        w = torch.empty_like(out)
+        _ham(1.0 + k)[0].apply(_fresh(k), w)
+        want.append(w)
+    busy = torch.zeros(1 << 26, device="cuda")
+    torch.cuda.synchronize()
+    for k in (1, 2, 0, 1):
+        with torch.cuda.stream(a):
+            for _ in range(20):
+                busy.add_(1.0)  # work in front of the copies
+            plan.update(_rows(k))
+            ham.set_coeffs((1.0 + k) * np.linspace(0.5, 1.5, nt))
+        with torch.cuda.stream(b):
+            graph.replay()
+        b.synchronize()
+        assert torch.equal(out, want[k])
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("count", [0, 1, 7, 8, 40])
 def test_update_many(gpu, count):
     """One thread, two threads and eight; a wrong op count fails and says so."""

@@ -1,7 +1,7 @@
 """Staged host-to-device copies and the marks that order later uses after them
 (tests/stage_check.cpp, over imitated streams; CPU only): several threads,
-streams that begin a capture or are destroyed after their copy, and more copies
-in flight than the ring holds."""
+streams that begin a capture or are destroyed after their copy, replays of
+captured graphs on other streams, and more copies in flight than the ring holds."""
 from __future__ import annotations
 
 import os
@@ -28,8 +28,9 @@ def checker(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("scenario", ["two_threads", "updater_under_capture", "ring_capture",
-                                      "ring_gone", "in_flight", "thread_ends", "refused"])
+@pytest.mark.parametrize("scenario", ["two_threads", "updater_under_capture",
+                                      "capture_on_own_stream", "update_after_capture",
+                                      "ring_capture", "ring_gone", "in_flight", "thread_ends", "refused"])
 def test_staging(checker, scenario):
     r = subprocess.run([str(checker), scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -34,7 +34,10 @@ StagePoint stage_point();
 // on that stream follow them anyway; the first use on another one waits on the
 // host until they have run (a device-side wait needs an event, which is a
 // packet for the device at every update, or recorded later on a stream that
-// may be under capture, or gone, by then).  Several threads may use an object.
+// may be under capture, or gone, by then).  A replay of a captured graph passes
+// no such place, on whatever stream it runs: a use under capture waits on its own
+// stream too, and from then on the object's copies are waited for where they are
+// queued.  Several threads may use an object.
 class StreamMark {
  public:
   StreamMark() = default;
@@ -45,6 +48,7 @@ class StreamMark {
     std::lock_guard<std::mutex> lock(m_);
     at_ = stage_point();
     st_ = st;
+    if (captured_) finish();
   }
   void clear() {
     std::lock_guard<std::mutex> lock(m_);
@@ -52,17 +56,25 @@ class StreamMark {
   }
   hipError_t wait(hipStream_t st) {
     std::lock_guard<std::mutex> lock(m_);
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(st, &cs);
+    if (e != hipSuccess) return e;
+    if (cs != hipStreamCaptureStatusNone) captured_ = true;
     // (each thread has a stream of its own behind hipStreamPerThread)
-    if (!at_.of || (st == st_ && st != hipStreamPerThread)) return hipSuccess;
-    at_.wait();
-    at_ = StagePoint{};
+    if (captured_ || st != st_ || st == hipStreamPerThread) finish();
     return hipSuccess;
   }
 
  private:
+  void finish() {
+    at_.wait();
+    at_ = StagePoint{};
+  }
+
   std::mutex m_;
   StagePoint at_;
   hipStream_t st_ = nullptr;
+  bool captured_ = false;
 };
 
 }  // namespace tqsv
