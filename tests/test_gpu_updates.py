@@ -175,3 +175,37 @@ def test_update_many(gpu, count):
     if count > 1:
         with pytest.raises(ValueError, match="repeated"):
             nat.update_plans([plans[0], plans[0]], [rows[0], rows[0]])
+
+
+def test_batch_with_some_generated_plans(gpu, capfd, monkeypatch):
+    """Plans that ask for generated kernels, behind one that does not: each
+    distinct pass is compiled once."""
+    import torch
+
+    import tyxonq_amd as tq
+    from tyxonq_amd import _native as nat
+    from tyxonq_amd.engine import lower
+    from tyxonq_amd.pauli import PauliSum
+
+    n, count = 6, 12
+    t = [torch.tensor(0.1 * q + 0.05, requires_grad=True) for q in range(n)]
+    c = tq.Circuit(n)
+    for q in range(n):
+        c.ry(q, t[q])
+    for q in range(n - 1):
+        c.cx(q, q + 1)
+    rows = lower(c, track_grad=True)[0].segments[0][1]
+    ham = nat.Ham(n, *PauliSum(n, [(1.0, [("Z", q), ("X", (q + 1) % n)]) for q in range(n)]
+                               + [(0.5, [("Z", q)]) for q in range(n)]).to_masks())
+    monkeypatch.setenv("TQSV_JIT_VERBOSE", "1")
+    res = []
+    for jit in ([-1] * count, [-1] + [1] * (count - 1)):
+        plans = [nat.Plan(n, rows, jit=j, min_qubits=nat.BATCH_QUBITS) for j in jit]
+        capfd.readouterr()
+        psis = [nat.new_state(n, 0) for _ in plans]
+        res += nat.Batch().adjoint(plans, [ham] * count, psis, [n] * count)
+        lines = [x.split("(hiprtc")[0] for x in capfd.readouterr().err.splitlines()
+                 if x.startswith("tqsv jit: pass") and "mode 2" in x]
+        assert len(lines) == len(set(lines))  # (one state tile: passes differ in their place)
+    for e, g in res[1:]:
+        assert e == res[0][0] and np.array_equal(g, res[0][1])

@@ -1344,9 +1344,12 @@ int tqsv_batch_adjoint(tqsv_batch* b, int nreq, tqsv_plan* const* plans, tqsv_ha
       if (!p->adj_built && std::find(build.begin(), build.end(), p) == build.end()) build.push_back(p);
     }
     if (!build.empty()) {
-      // (generated kernels, forced by TQSV_JIT, are compiled one plan at a time)
+      // one plan at a time if any compiles kernels (asked for by its options or by
+      // TQSV_JIT): for the calling thread's device, and once per distinct pass
+      bool serial = false;
+      for (const tqsv_plan* p : build) serial = serial || jit_policy(p->jit_req, p->n, 1, 64);
       auto emit = [&](int i) { return plan_emit_adjoint(build[(size_t)i]); };
-      if (jit_policy(build[0]->jit_req, BATCH_QUBITS, 1, 64)) {
+      if (serial) {
         for (int i = 0; !rc && i < (int)build.size(); ++i) rc = emit(i);
       } else {
         rc = parallel_calls((int)build.size(), emit);
