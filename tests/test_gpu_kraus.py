@@ -74,6 +74,18 @@ def test_chain_edges():
         nat.kraus_chain(v, [(0, [], 0.5)])
 
 
+def test_operators_of_another_size_are_refused():
+    """Nothing is cut off or made up: the state stays as it is."""
+    from tyxonq_amd import _native as nat
+
+    v = to_gpu(rand_state(np.random.default_rng(2), 6))
+    before = to_np(v)
+    for bad in (np.eye(4), np.eye(3), np.eye(1)):
+        with pytest.raises(ValueError, match="2x2"):
+            nat.kraus_chain(v, [(0, [np.eye(2), bad], 0.5)])
+    np.testing.assert_array_equal(to_np(v), before)
+
+
 # below, at and above one chunk, several blocks, and chunks beyond the grid
 @pytest.mark.parametrize("n", [1, 7, 12, 13, 18, 25])
 def test_expect_z_all(n):

@@ -320,7 +320,7 @@ def kraus_chain(psi, channels: Sequence[tuple]) -> None:
     c = len(channels)
     if c == 0:
         return
-    mats = [np.asarray(K, dtype=np.complex128).reshape(-1)[:4] for _, ks, _ in channels for K in ks]
+    mats = [np.asarray(K, dtype=np.complex128).reshape(-1) for _, ks, _ in channels for K in ks]
     if any(m.size != 4 for m in mats):
         raise ValueError("Kraus operators must be 2x2")
     ops = np.ascontiguousarray(np.stack(mats)) if mats else np.zeros((1, 4), dtype=np.complex128)
