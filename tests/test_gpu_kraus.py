@@ -86,6 +86,28 @@ def test_operators_of_another_size_are_refused():
     np.testing.assert_array_equal(to_np(v), before)
 
 
+def test_long_tables_are_given_back():
+    """16 MiB of operators on the device; what stays is bounded by a 10-qubit
+    matrix (8 MiB) in each of two slots, filled here first."""
+    import torch
+
+    from tyxonq_amd import _native as nat
+
+    v = to_gpu(rand_state(np.random.default_rng(4), 10))
+    for _ in range(2):
+        nat.apply_kq(v, list(range(10)), np.eye(1 << 10))
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    # 2^18 operators of weight 1e-18, then the identity, which is chosen
+    ks = [np.array([[0, 1], [1, 0]]) * 1e-9] * (1 << 18) + [np.eye(2)]
+    want = to_np(v)
+    for _ in range(2):
+        nat.kraus_chain(v, [(3, ks, 0.5)])
+    torch.cuda.synchronize()
+    assert np.linalg.norm(to_np(v) - want) <= 8 * 2.0 ** -24
+    assert free - torch.cuda.mem_get_info()[0] <= 4 << 20
+
+
 # below, at and above one chunk, several blocks, and chunks beyond the grid
 @pytest.mark.parametrize("n", [1, 7, 12, 13, 18, 25])
 def test_expect_z_all(n):

@@ -42,7 +42,10 @@ int scratch(size_t ndoubles, double** out) {
 // page-locked buffer, its device copy and the event after the last kernel that
 // reads it.  A slot is taken again only when that event has passed, so calls
 // need no stream synchronisation, on whatever streams the thread uses.  Slots
-// grow to the largest call (8 MiB for a 10-qubit matrix) and go with the thread.
+// grow to the largest call, up to that of a 10-qubit matrix, and go with the
+// thread; what a longer table took (a Kraus chain of 10^5 operators) is waited
+// for and given back.
+constexpr size_t kUploadKeep = (8u << 20) + (64u << 10);
 struct Upload {
   unsigned char* h = nullptr;
   unsigned char* d = nullptr;
@@ -100,6 +103,7 @@ hipError_t upload_done(Upload* u, hipStream_t st) {
     u->busy = true;
   else
     (void)hipStreamSynchronize(st);
+  if (u->cap > kUploadKeep) u->drop();
   return e;
 }
 
