@@ -42,6 +42,23 @@ def test_kq_against_oracle(n, qubits, offset):
     np.testing.assert_array_equal(to_np(src), to_np(to_gpu(v)))
 
 
+# index bits in each order: one thread's work with bit 0 a target (n = 3) and not
+# (n = 4); LDS tiles at two targets below bit 5, one tile and several; bit 5 itself;
+# part of a work-group
+@pytest.mark.parametrize("n,bits", [
+    (3, [0, 1, 2]), (3, [2, 0, 1]), (4, [3, 1, 2]), (4, [0, 3, 2]), (9, [8, 0, 4]),
+    (11, [1, 2, 3]), (12, [1, 2, 3]), (12, [0, 11, 4]), (12, [4, 5, 11]), (12, [5, 0, 6]),
+    (12, [11, 9, 10]), (15, [14, 4, 3]), (16, [2, 0, 1]), (17, [5, 16, 1]), (18, [17, 3, 10])])
+def test_three_targets(n, bits):
+    from tyxonq_amd import _native as nat
+
+    rng = np.random.default_rng(n + bits[0])
+    v, U = to_gpu(rand_state(rng, n)), rand_unitary(rng, 8)
+    ref = O.apply_kqubit(to_np(v), U, [n - 1 - b for b in bits], n)
+    # unit-norm rows: 16 FP32 products and sums of random sign, 2^-24 each
+    assert np.linalg.norm(to_np(nat.apply_kq(v, bits, U)) - ref) <= 4 * 2.0 ** -24 * np.sqrt(8.0)
+
+
 def test_kq_calls_in_flight_on_two_streams():
     """The tables of a call are staged until its kernel has run."""
     import torch

@@ -227,57 +227,47 @@ int tqsv_apply_kq(const void* psi, void* out, int n, int k, const int* bits, con
     pos[b] = (uint32_t)bits[b];
   }
   if ((rc = refuse_capture(S(stream), "tqsv_apply_kq"))) return rc;
-  // Matrix cores for 3 <= k <= 10 with enough other bits for a tile and 16-byte
-  // aligned states; k = 3 runs as k = 4 with the lowest other bit as an
-  // untouched target (U x I: twice the products, but 27 qubits are HBM-bound
-  // either way, 1.47 -> 0.41 ms).  The general kernel keeps what has no such
-  // tile (n below 12, or n - k below 6 for k >= 6: at most 2^15 amplitudes, a
-  // launch's latency) and states at 8-byte alignment.
-  KqGeo geo;
-  std::vector<uint32_t> tb(pos);
-  if (k == 3 && n > 3) {
-    uint32_t b = 0;
-    while ((seen >> b) & 1ull) ++b;
-    tb.push_back(b);
-  }
-  const int kk = (int)tb.size();
   const bool aligned = ((reinterpret_cast<uintptr_t>(psi) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
-  const bool mfma = aligned && kq_mfma_geo(n, kk, tb.data(), &geo);
+  // k = 3: HBM-bound in vector arithmetic, the matrix in the launch's arguments
+  if (k == 3 && aligned) {
+    Mat8f u;
+    for (int j = 0; j < 128; ++j) u.v[j] = (float)U[j];
+    TQSV_HIP(k_apply_3q_to(CF(psi), F(out), n, bits, u, S(stream)));
+    return 0;
+  }
+  // Matrix cores for 4 <= k <= 10 with enough other bits for a tile and 16-byte
+  // aligned states.  The general kernel keeps what has no such tile (n below 12,
+  // or n - k below 6 for k >= 6: at most 2^15 amplitudes, a launch's latency) and
+  // states at 8-byte alignment.
+  KqGeo geo;
+  const bool mfma = aligned && kq_mfma_geo(n, k, pos.data(), &geo);
   const size_t K = (size_t)1 << k;
-  const size_t KK = (size_t)1 << kk;
-  const size_t bytes = mfma ? KK * KK * sizeof(float2)
+  const size_t bytes = mfma ? K * K * sizeof(float2)
                             : K * K * sizeof(float2) + K * sizeof(uint64_t) + (size_t)k * sizeof(uint32_t);
   Upload* up = nullptr;
   if ((rc = upload_slot(bytes, &up))) return rc;
   float2* hu = reinterpret_cast<float2*>(up->h);
   if (mfma) {
     // row/column number by ascending target bits -> index of U (first target
-    // most significant); the added bit of k = 3 gives the block (bit + 1) - 1
-    std::vector<uint32_t> order(kk);
-    for (int b = 0; b < kk; ++b) order[b] = (uint32_t)b;
-    std::sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return tb[x] < tb[y]; });
-    std::vector<uint32_t> ui(KK), extra(KK);
-    for (size_t j = 0; j < KK; ++j) {
-      uint32_t v = 0, e = 0;
-      for (int b = 0; b < kk; ++b)
-        if ((j >> b) & 1u) {
-          if (order[b] < (uint32_t)k)
-            v |= 1u << (k - 1 - order[b]);
-          else
-            e = 1;
-        }
+    // most significant)
+    std::vector<uint32_t> order(k);
+    for (int b = 0; b < k; ++b) order[b] = (uint32_t)b;
+    std::sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return pos[x] < pos[y]; });
+    std::vector<uint32_t> ui(K);
+    for (size_t j = 0; j < K; ++j) {
+      uint32_t v = 0;
+      for (int b = 0; b < k; ++b)
+        if ((j >> b) & 1u) v |= 1u << (k - 1 - order[b]);
       ui[j] = v;
-      extra[j] = e;
     }
-    const size_t chunk = kk < 6 ? KK : 64;
+    const size_t chunk = k < 6 ? K : 64;
     float2* o = hu;
-    for (size_t m = 0; m < KK / 16; ++m)
-      for (size_t c = 0; c < KK; c += chunk)
+    for (size_t m = 0; m < K / 16; ++m)
+      for (size_t c = 0; c < K; c += chunk)
         for (size_t t = 0; t < chunk; ++t)
           for (size_t r = 0; r < 16; ++r, ++o) {
-            const size_t row = 16 * m + r, col = c + t;
-            const double* e = U + 2 * ((size_t)ui[row] * K + ui[col]);
-            *o = extra[row] == extra[col] ? make_float2((float)e[0], (float)e[1]) : make_float2(0.f, 0.f);
+            const double* e = U + 2 * ((size_t)ui[16 * m + r] * K + ui[c + t]);
+            *o = make_float2((float)e[0], (float)e[1]);
           }
   } else {
     for (size_t e = 0; e < K * K; ++e) hu[e] = make_float2((float)U[2 * e], (float)U[2 * e + 1]);
@@ -293,7 +283,7 @@ int tqsv_apply_kq(const void* psi, void* out, int n, int k, const int* bits, con
   if (e == hipSuccess) {
     const float2* dU = reinterpret_cast<const float2*>(up->d);
     const uint64_t* dOff = reinterpret_cast<const uint64_t*>(dU + K * K);
-    e = mfma ? k_apply_kq_mfma(CF(psi), F(out), kk, geo, dU, S(stream))
+    e = mfma ? k_apply_kq_mfma(CF(psi), F(out), k, geo, dU, S(stream))
              : k_apply_kq(CF(psi), F(out), n, k, reinterpret_cast<const uint32_t*>(dOff + K), dOff,
                           dU, S(stream));
   }

@@ -66,7 +66,11 @@ hipError_t k_stage_copy(void* dst, const void* src, size_t bytes, uint64_t* word
                         uint64_t number, hipStream_t st);
 hipError_t k_apply_kq(const float2* psi, float2* out, int n, int k, const uint32_t* bitpos,
                       const uint64_t* off, const float2* U, hipStream_t st);
-// Matrix-core form of the same (tqsv_kq.hip): tiles of 2^KQ_TILE_BITS
+// k = 3 on 16-byte aligned states: bits[0] the most significant index of U
+struct Mat8f { float v[128]; };  // row-major re/im
+hipError_t k_apply_3q_to(const float2* psi, float2* out, int n, const int* bits, const Mat8f& u,
+                         hipStream_t st);
+// Matrix-core form of the same for k >= 4 (tqsv_kq.hip): tiles of 2^KQ_TILE_BITS
 // amplitudes over the lowest targets and the lowest other index bits.
 constexpr int KQ_TILE_BITS = 12;
 struct KqGeo {
