@@ -184,7 +184,8 @@ template <typename IDX>
 __device__ __forceinline__ bool q_on(const QuadGeo<IDX>& G, int s, IDX cm, IDX cv, bool ton) {
   return ton && ((gs_reg(G, s) ^ G.gq) & cm & G.rmask) == (cv & G.rmask);
 }
-template <int K, typename IDX>
+// (products with the zeros of a TYPE are left out: an infinity times 0 is NaN)
+template <int K, uint32_t TYPE, typename IDX>
 __device__ __forceinline__ void qu1(float2 (&a)[NR], const M2f& u, const QuadGeo<IDX>& G, IDX cm,
                                     IDX cv, bool ton) {
   if constexpr (K >= 2) {
@@ -194,7 +195,7 @@ __device__ __forceinline__ void qu1(float2 (&a)[NR], const M2f& u, const QuadGeo
       const int s1 = s | (1 << (K - 2));
       const bool on = q_on(G, s, cm, cv, ton);
       float2 y0, y1;
-      mul2<U1_GENERAL>(u, a[s], a[s1], y0, y1);
+      mul2<TYPE>(u, a[s], a[s1], y0, y1);
       a[s] = sel2(on, y0, a[s]);
       a[s1] = sel2(on, y1, a[s1]);
     }
@@ -206,8 +207,14 @@ __device__ __forceinline__ void qu1(float2 (&a)[NR], const M2f& u, const QuadGeo
     for (int s = 0; s < NR; ++s) {
       const bool on = q_on(G, s, cm, cv, ton);
       const float2 x = a[s], p = qx2<1 << K>(a[s]);
-      const float2 y = make_float2(dr * x.x - di * x.y + er * p.x - ei * p.y,
-                                   dr * x.y + di * x.x + er * p.y + ei * p.x);
+      float2 y;
+      if constexpr (TYPE == U1_REAL)
+        y = make_float2(dr * x.x + er * p.x, dr * x.y + er * p.y);
+      else if constexpr (TYPE == U1_RXLIKE)
+        y = make_float2(dr * x.x - ei * p.y, dr * x.y + ei * p.x);
+      else
+        y = make_float2(dr * x.x - di * x.y + er * p.x - ei * p.y,
+                        dr * x.y + di * x.x + er * p.y + ei * p.x);
       a[s] = sel2(on, y, x);
     }
   }
@@ -351,12 +358,11 @@ __device__ __forceinline__ void qpgrp(float2 (&a)[NR], const float2 (&p)[NR], ui
     if ((((Mi | Mj) >> (4 * s)) & 15u) == 0) continue;  // uniform: no lane's slot is active
     const bool i = ((mi >> (4 * s)) & 1u) != 0, j = ((mj >> (4 * s)) & 1u) != 0;
     const uint32_t sg = tsign ^ (((sm >> (4 * s)) & 1u) << 31);
-    const float cm = i || j ? cm1 : 0.f;
-    const float ur = flip(i ? ujr : (j ? uir : 0.f), sg), ui = flip(i ? uji : (j ? uii : 0.f), sg);
+    const float ur = flip(i ? ujr : uir, sg), ui = flip(i ? uji : uii, sg);
     const float2 x = a[s], w = p[s];
-    const float tr = fmaf(-ui, w.y, fmaf(cm, x.x, ur * w.x));
-    const float ti = fmaf(ui, w.x, fmaf(cm, x.y, ur * w.y));
-    a[s] = make_float2(x.x + tr, x.y + ti);
+    const float tr = fmaf(-ui, w.y, fmaf(cm1, x.x, ur * w.x));
+    const float ti = fmaf(ui, w.x, fmaf(cm1, x.y, ur * w.y));
+    a[s] = sel2(i || j, make_float2(x.x + tr, x.y + ti), x);
   }
 }
 
@@ -490,16 +496,28 @@ __device__ __forceinline__ void run_step(const step_t& h, cw_t w, float2 (&a)[NR
       const IDX cm = widx<IDX>(h[4], h[5]), cv = widx<IDX>(h[6], h[7]);
       const bool ton = (G.gb & cm) == (cv & ~G.rmask);
       const M2f u{F(8), F(9), F(10), F(11), F(12), F(13), F(14), F(15)};
-#define TQSV_QU(K)                                            \
-  case K:                                                     \
-    qu1<K, IDX>(a, u, G, cm, cv, ton);                        \
-    if constexpr (DUAL) qu1<K, IDX>(b, u, G, cm, cv, ton);    \
-    TQSV_ARM_END("u1", K);                                    \
+#define TQSV_QU(K, TY)                                              \
+  case 4 * K + TY:                                                  \
+    qu1<K, TY, IDX>(a, u, G, cm, cv, ton);                          \
+    if constexpr (DUAL) qu1<K, TY, IDX>(b, u, G, cm, cv, ton);      \
+    TQSV_ARM_END("u1", 4 * K + TY);                                 \
     break;
-      switch (h[1]) {
-        TQSV_QU(0) TQSV_QU(1) TQSV_QU(2) TQSV_QU(3) TQSV_QU(4)
-        default: break;
+#define TQSV_QUK(K) TQSV_QU(K, 1) TQSV_QU(K, 2)
+      const uint32_t arm = 4u * h[1] + h[2];
+      // (the other types' arms are placed after the kernel's: in line they took 1 us
+      // of 50 from 66 general matrices at 11 qubits)
+      if (__builtin_expect(h[2] == U1_GENERAL, 1)) {
+        switch (arm) {
+          TQSV_QU(0, 0) TQSV_QU(1, 0) TQSV_QU(2, 0) TQSV_QU(3, 0) TQSV_QU(4, 0)
+          default: break;
+        }
+      } else {
+        switch (arm) {
+          TQSV_QUK(0) TQSV_QUK(1) TQSV_QUK(2) TQSV_QUK(3) TQSV_QUK(4)
+          default: break;
+        }
       }
+#undef TQSV_QUK
 #undef TQSV_QU
       break;
     }
@@ -613,11 +631,10 @@ __device__ __forceinline__ void run_step(const step_t& h, cw_t w, float2 (&a)[NR
               if ((((Mi | Mj) >> (4 * s)) & 15u) == 0) continue;
               const bool i = ((mi >> (4 * s)) & 1u) != 0, j = ((mj >> (4 * s)) & 1u) != 0;
               const uint32_t sg = ts ^ (((sm >> (4 * s)) & 1u) << 31);
-              const float wr = flip(i ? vjr : (j ? vir : 0.f), sg);
-              const float wi = flip(i ? vji : (j ? vii : 0.f), sg);
+              const float wr = flip(i ? vjr : vir, sg), wi = flip(i ? vji : vii, sg);
               // Im(conj(l) w a) = l.x (w.r a.y + w.i a.x) - l.y (w.r a.x - w.i a.y)
-              v = fmaf(b[s].x, wr * p[s].y + wi * p[s].x, v);
-              v = fmaf(-b[s].y, wr * p[s].x - wi * p[s].y, v);
+              const float t = fmaf(b[s].x, wr * p[s].y + wi * p[s].x, v);
+              v = i || j ? fmaf(-b[s].y, wr * p[s].x - wi * p[s].y, t) : v;
             }
           }
           put_red(v, acc, nred, slot);
