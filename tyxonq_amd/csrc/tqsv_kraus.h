@@ -25,9 +25,11 @@ hipError_t k_kraus_apply(float2* psi, int n, int bit, int next, const KrausItem*
 // psi /= sqrt(sum of rho00 + rho11 in `in`) unless that is 0
 hipError_t k_kraus_normalise(float2* psi, int n, const double* in, hipStream_t st);
 
-// out[b] = <Z_b> for every index bit; partials: zall_doubles(n) doubles
+// <Z_b> for every index bit b at (*result)[b], in `partials` (zall_doubles(n)
+// doubles) when one block sums the state, else in out
 size_t zall_doubles(int n);
-hipError_t k_zall(const float2* psi, int n, double* partials, double* out, hipStream_t st);
+hipError_t k_zall(const float2* psi, int n, double* partials, double* out, const double** result,
+                  hipStream_t st);
 
 }  // namespace tqsv
 

@@ -298,12 +298,18 @@ static uint32_t zall_blocks(int n) {
 }
 size_t zall_doubles(int n) { return (size_t)zall_blocks(n) * ZVALS; }
 
-hipError_t k_zall(const float2* psi, int n, double* partials, double* out, hipStream_t st) {
+hipError_t k_zall(const float2* psi, int n, double* partials, double* out, const double** result,
+                  hipStream_t st) {
   const dim3 G(zall_blocks(n)), B(BLK);
   if (n > ZB + ZGRID)
     hipLaunchKernelGGL(zall_kernel<true>, G, B, 0, st, psi, 1ull << n, 1u << (n - ZB - ZGRID), partials);
   else
     hipLaunchKernelGGL(zall_kernel<false>, G, B, 0, st, psi, 1ull << n, 1u, partials);
+  if (n <= ZB) {  // one block, and every bit is a low one: its sums are the result
+    *result = partials;
+    return hipGetLastError();
+  }
+  *result = out;
   hipLaunchKernelGGL(zall_final_kernel, dim3((uint32_t)n), B, 0, st, partials, zall_blocks(n), out);
   return hipGetLastError();
 }
