@@ -127,3 +127,26 @@ def test_expect_z_all(n):
     idx = np.arange(1 << n)
     ref = [np.sum(p * (1 - 2 * ((idx >> b) & 1))) for b in range(n)]
     np.testing.assert_allclose(nat.expect_z_all(v), ref, atol=1e-12)  # FP64 products and sums
+
+
+@pytest.mark.parametrize("n", [1, 5, 13])
+def test_run_with_one_and_with_every_qubit_measured(n):
+    """The same values from the reduction of one qubit and the sweep of all."""
+    import tyxonq_amd as tq
+    from tyxonq_amd.engine import StatevectorEngine
+
+    def run(measured):
+        c = tq.Circuit(n)
+        for q in range(n):
+            c.ry(q, 0.3 + 0.2 * q)
+        for q in measured:
+            c.measure_z(q)
+        return StatevectorEngine().run(c, shots=0)["expectations"]
+
+    every = run(range(n))
+    for q in range(n):
+        one = run([q, q])
+        assert list(one) == [f"Z{q}"]
+        # FP64 sums of the same probabilities; n rotations in FP32
+        assert one[f"Z{q}"] == pytest.approx(every[f"Z{q}"], abs=1e-12)
+        assert one[f"Z{q}"] == pytest.approx(math.cos(0.3 + 0.2 * q), abs=n * 2.0 ** -23)
