@@ -117,7 +117,11 @@ int tqsv_reduce_blocks(int n);
 int tqsv_expect_z_dev(const void* psi, int n, int bit, double* partials_dev, double* out_dev,
                       void* stream);
 
-/* out[b] = <Z_b> for every index bit b < n (host), in one sweep. */
+/* tqsv_expect_z with FP64 products as well as sums. */
+int tqsv_expect_z_fp64(const void* psi, int n, int bit, double* out, void* stream);
+
+/* out[b] = <Z_b> for every index bit b < n (host), in one sweep, FP64 products
+ * and sums. */
 int tqsv_expect_z_all(const void* psi, int n, double* out, void* stream);
 
 /* A chain of stochastic one-qubit Kraus channels (kernels/statevector.py:

@@ -108,6 +108,7 @@ _SIGS = {
     "tqsv_scale": (_I, [_P, _I, _D, _D, _P]),
     "tqsv_norm2": (_I, [_P, _I, _DP, _P]),
     "tqsv_expect_z": (_I, [_P, _I, _I, _DP, _P]),
+    "tqsv_expect_z_fp64": (_I, [_P, _I, _I, _DP, _P]),
     "tqsv_reduce_blocks": (_I, [_I]),
     "tqsv_expect_z_dev": (_I, [_P, _I, _I, _P, _P, _P]),
     "tqsv_expect_z_all": (_I, [_P, _I, _DP, _P]),
@@ -412,6 +413,14 @@ def expect_z(psi, bit: int) -> float:
     _check(
         load().tqsv_expect_z(_ptr(psi), _nqubits(psi), int(bit), ctypes.byref(out), stream_ptr())
     )
+    return out.value
+
+
+def expect_z_fp64(psi, bit: int) -> float:
+    """expect_z with FP64 products, as expect_z_all's."""
+    out = ctypes.c_double(0.0)
+    _check(load().tqsv_expect_z_fp64(_ptr(psi), _nqubits(psi), int(bit), ctypes.byref(out),
+                                     stream_ptr()))
     return out.value
 
 

@@ -415,6 +415,14 @@ int tqsv_expect_z(const void* psi, int n, int bit, double* out, void* stream) {
   return reduce_prob_to_host(CF(psi), n, 1, bit, out, S(stream));
 }
 
+int tqsv_expect_z_fp64(const void* psi, int n, int bit, double* out, void* stream) {
+  int rc = check_state(psi, n, "tqsv_expect_z_fp64");
+  if (rc) return rc;
+  if ((rc = check_bit(bit, n, "tqsv_expect_z_fp64"))) return rc;
+  if (!out) return fail(TQSV_EINVAL, "tqsv_expect_z_fp64: out is NULL");
+  return reduce_prob_to_host(CF(psi), n, 3, bit, out, S(stream));
+}
+
 int tqsv_reduce_blocks(int n) { return n < 1 || n > 34 ? 0 : (int)reduce_grid(n); }
 
 int tqsv_expect_z_dev(const void* psi, int n, int bit, double* partials_dev, double* out_dev,

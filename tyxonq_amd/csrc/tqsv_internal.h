@@ -89,7 +89,8 @@ bool kq_mfma_geo(int n, int k, const uint32_t* bits, KqGeo* geo);
 hipError_t k_apply_kq_mfma(const float2* psi, float2* out, int k, const KqGeo& g, const float2* A,
                            hipStream_t st);
 hipError_t k_probs(const float2* psi, int n, double* out, hipStream_t st);
-// blockwise FP64 partial sums: mode 0 = |psi|^2, 1 = |psi|^2 (-1)^{bit}, 2 = |psi|^2 [bit==keep]
+// blockwise FP64 partial sums: mode 0 = |psi|^2, 1 = |psi|^2 (-1)^{bit}, 2 = |psi|^2 [bit==keep],
+// 3 = as 1 with FP64 products
 uint32_t reduce_grid(int n);
 hipError_t k_reduce_prob(const float2* psi, int n, int mode, int bit, double* partials,
                          hipStream_t st);

@@ -186,6 +186,20 @@ __global__ __launch_bounds__(BLK) void reduce_prob_kernel(const float2* psi, uin
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
+// mode 1 with FP64 products (28 qubits: 394 us, with FP32 products 408)
+__global__ __launch_bounds__(BLK) void reduce_z_fp64_kernel(const float2* psi, uint64_t dim,
+                                                            uint32_t bit, double* partials) {
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  double acc = 0.0;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < dim; i += stride) {
+    const float2 v = psi[i];
+    const double p = (double)v.x * v.x + (double)v.y * v.y;
+    acc += (i >> bit) & 1ull ? -p : p;
+  }
+  const double s = block_sum(acc);
+  if (threadIdx.x == 0) partials[blockIdx.x] = s;
+}
+
 __global__ __launch_bounds__(BLK) void final_sum_kernel(const double* partials, uint32_t ngroups,
                                                         uint32_t nred, double* out) {
   const uint32_t r = blockIdx.x;
@@ -603,6 +617,11 @@ uint32_t reduce_grid(int n) {
 hipError_t k_reduce_prob(const float2* psi, int n, int mode, int bit, double* partials,
                          hipStream_t st) {
   const uint64_t dim = 1ull << n;
+  if (mode == 3) {
+    hipLaunchKernelGGL(reduce_z_fp64_kernel, dim3(reduce_grid(n)), dim3(BLK), 0, st, psi, dim,
+                       (uint32_t)bit, partials);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(reduce_prob_kernel, dim3(reduce_grid(n)), dim3(BLK), 0, st, psi, dim, mode,
                      (uint32_t)bit, partials);
   return hipGetLastError();

@@ -586,12 +586,12 @@ class StatevectorEngine:
                     "metadata": {"shots": shots, "backend": self.backend.name,
                                  "three_level": bool(kwargs.get("three_level", False))}}
         expectations: Dict[str, float] = {}
-        # one qubit by its own reduction (28 qubits: 411 us, every qubit 502 us)
+        # one qubit by its own reduction (28 qubits: 394 us, every qubit 499)
         zs = nat.expect_z_all(psi) if len(set(measures)) > 1 else None
         for q in measures:
             if not 0 <= q < n:
                 raise ValueError(f"measured qubit {q} out of range for n={n}")
-            val = nat.expect_z(psi, n - 1 - q) if zs is None else zs[n - 1 - q]
+            val = nat.expect_z_fp64(psi, n - 1 - q) if zs is None else zs[n - 1 - q]
             if z_atten is not None:
                 val *= z_atten[q]
             expectations[f"Z{q}"] = float(val)
