@@ -263,14 +263,18 @@ int tqsv_apply_kq(const void* psi, void* out, int n, int k, const int* bits, con
       ui[j] = v;
     }
     const size_t chunk = k < 6 ? K : 64;
+    // along U's rows: 16 of them at a time are 16 lines of one cache set (k = 10:
+    // 0.75 to 2.0 ms, depending on the targets, so 0.48 to 0.64)
     float2* o = hu;
     for (size_t m = 0; m < K / 16; ++m)
-      for (size_t c = 0; c < K; c += chunk)
-        for (size_t t = 0; t < chunk; ++t)
-          for (size_t r = 0; r < 16; ++r, ++o) {
-            const double* e = U + 2 * ((size_t)ui[16 * m + r] * K + ui[c + t]);
-            *o = make_float2((float)e[0], (float)e[1]);
+      for (size_t c = 0; c < K; c += chunk, o += 16 * chunk)
+        for (size_t r = 0; r < 16; ++r) {
+          const double* row = U + 2 * (size_t)ui[16 * m + r] * K;
+          for (size_t t = 0; t < chunk; ++t) {
+            const double* e = row + 2 * (size_t)ui[c + t];
+            o[16 * t + r] = make_float2((float)e[0], (float)e[1]);
           }
+        }
   } else {
     for (size_t e = 0; e < K * K; ++e) hu[e] = make_float2((float)U[2 * e], (float)U[2 * e + 1]);
     uint64_t* off = reinterpret_cast<uint64_t*>(hu + K * K);

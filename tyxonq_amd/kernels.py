@@ -60,7 +60,7 @@ def _as_state(state: Any, num_qubits: int):
 def _resolved(t: Any):
     """t with a pending conjugation or sign change written out: the kernels read
     the memory, and reshape, contiguous and .to() keep those flags."""
-    return t.resolve_conj().resolve_neg()
+    return t.resolve_conj().resolve_neg() if t.is_conj() or t.is_neg() else t
 
 
 def _mat(m: Any, dim: int) -> np.ndarray:
