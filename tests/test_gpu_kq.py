@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 # (n, qubits): the smallest tile of each k and one bit below it (general
 # kernel), targets lowest, highest, interleaved and in descending order, chunks
-# and row blocks of k >= 7, several tiles per work-group (19 qubits at k = 4)
+# and row blocks of k >= 7, several tiles (19 qubits at k = 4: a work-group each;
+# work-groups with several tiles are in test_work_groups_with_several_tiles)
 CASES = [
     (3, [2, 0, 1]), (11, [0, 5, 10]), (12, [11, 10, 9]), (12, [0, 1, 2]),
     (11, [3, 1, 9, 4]), (12, [3, 1, 9, 4]), (12, [8, 9, 10, 11]), (19, [0, 18, 7, 3]),
@@ -57,6 +58,36 @@ def test_three_targets(n, bits):
     ref = O.apply_kqubit(to_np(v), U, [n - 1 - b for b in bits], n)
     # unit-norm rows: 16 FP32 products and sums of random sign, 2^-24 each
     assert np.linalg.norm(to_np(nat.apply_kq(v, bits, U)) - ref) <= 4 * 2.0 ** -24 * np.sqrt(8.0)
+
+
+# more work than the grid of 1024 (16384 for k = 3): 2 and 4 tiles per work-group,
+# U kept in registers over them; k >= 7: 2 tiles and 8 (interleaved over the XCDs),
+# and 4 pieces of work per work-group
+@pytest.mark.parametrize("n,qubits", [
+    (23, [22, 3, 11, 0]), (24, [5, 23, 0, 12, 7]), (24, [23, 1, 8, 22, 15, 4]),
+    (14, [13, 0, 6, 2, 9, 11, 4]), (16, [1, 15, 3, 8, 12, 0, 6]),
+    (24, [2, 23, 10, 0, 17, 21, 6]), (24, [0, 22, 4, 18, 9, 13, 23, 2]),
+    (27, [26, 24, 25])])
+def test_work_groups_with_several_tiles(n, qubits):
+    import torch
+
+    from tyxonq_amd import kernels as K
+
+    k, rng = len(qubits), np.random.default_rng(n + len(qubits))
+    torch.manual_seed(n + k)
+    v = torch.randn(1 << n, dtype=torch.complex64, device="cuda") * 2.0 ** (-n / 2)
+    U = rand_unitary(rng, 1 << k)
+    out = K.apply_kqubit_unitary(v, U, qubits, n)
+    # complex128 products in plain torch, 2^22 amplitudes at a time (targets first)
+    perm = list(qubits) + [a for a in range(n) if a not in qubits]
+    x = v.reshape((2,) * n).permute(perm).reshape(1 << k, -1)
+    y = out.reshape((2,) * n).permute(perm).reshape(1 << k, -1)
+    Ut, d2, r2 = torch.tensor(U, device="cuda"), 0.0, 0.0
+    for xs, ys in zip(x.split(1 << (22 - k), 1), y.split(1 << (22 - k), 1)):
+        ref = Ut @ xs.to(torch.complex128)
+        d2 += float((ys.to(torch.complex128) - ref).abs().square().sum())
+        r2 += float(ref.abs().square().sum())
+    assert d2 ** 0.5 <= 4 * 2.0 ** -24 * np.sqrt(2.0 ** k) * r2 ** 0.5
 
 
 def test_kq_calls_in_flight_on_two_streams():
