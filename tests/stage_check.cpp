@@ -98,6 +98,8 @@ hipError_t use(hipStream_t s, const char* what) {
   return hipSuccess;
 }
 std::function<void()> g_after_event_create;  // test hook
+int g_device = 0;
+std::atomic<int> g_allocations{0};
 
 }  // namespace
 
@@ -108,10 +110,11 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
 }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hipSuccess; }
 hipError_t hipGetDevice(int* d) {
-  *d = 0;
+  *d = g_device;
   return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned int) {
+  ++g_allocations;
   *p = std::aligned_alloc(4096, (n + 4095) / 4096 * 4096);
   return hipSuccess;
 }
@@ -378,6 +381,20 @@ void thread_ends() {
   expect(all(got, 9), "the table was read before its copy");
 }
 
+// a thread that goes back and forth between devices keeps its ring
+void two_devices() {
+  Stream s[2];
+  uint32_t dev[2] = {0, 0};
+  for (uint32_t k = 1; k <= 20; ++k) {
+    g_device = (int)(k % 2);
+    expect(stage_copy(&dev[g_device], &k, 4, H(s[g_device])) == 0, "refused");
+  }
+  s[0].drain();
+  s[1].drain();
+  expect(dev[0] == 20 && dev[1] == 19, "a copy is wrong");
+  expect(g_allocations == 1, "the ring was allocated again");
+}
+
 // refused on a stream under capture
 void refused() {
   Stream a;
@@ -399,6 +416,7 @@ int main(int argc, char** argv) {
   else if (w == "ring_gone") ring(true);
   else if (w == "in_flight") in_flight();
   else if (w == "thread_ends") thread_ends();
+  else if (w == "two_devices") two_devices();
   else if (w == "refused") refused();
   else return 2;
   if (g_fault) return 1;

@@ -30,7 +30,8 @@ def checker(tmp_path_factory):
 
 @pytest.mark.parametrize("scenario", ["two_threads", "updater_under_capture",
                                       "capture_on_own_stream", "update_after_capture",
-                                      "ring_capture", "ring_gone", "in_flight", "thread_ends", "refused"])
+                                      "ring_capture", "ring_gone", "in_flight", "thread_ends",
+                                      "two_devices", "refused"])
 def test_staging(checker, scenario):
     r = subprocess.run([str(checker), scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -48,7 +48,6 @@ constexpr size_t kQuarter = kRing / 4;   // larger copies go from the caller's m
 struct Ring {
   unsigned char* base = nullptr;  // the ring, then the words of the tickets
   size_t head = 0;
-  int dev = -1;
   std::shared_ptr<StageTickets> tickets;
   uint64_t next = 1;              // numbers start at 1: a word of 0 holds none
   uint64_t latest = 0;            // first number of the last copy
@@ -56,8 +55,8 @@ struct Ring {
     uint64_t first = 1, last = 0;
   } quarter[4];                   // numbers of each quarter's copies
 
-  int open(int device) {
-    drop();
+  // (portable memory: one ring serves whichever devices the thread uses)
+  int open() {
     const size_t words = StageTickets::kWords * sizeof(uint64_t);
     auto t = std::make_shared<StageTickets>();
     // (another thread may be capturing: an allocation is no part of that)
@@ -73,10 +72,9 @@ struct Ring {
     t->word = reinterpret_cast<uint64_t*>(base + kRing);
     std::memset(t->word, 0, words);
     tickets = std::move(t);
-    dev = device;
     return 0;
   }
-  void drop() {
+  ~Ring() {
     if (!base) return;
     tickets->wait(next > StageTickets::kWords ? next - StageTickets::kWords : 1, next - 1);
     {
@@ -84,13 +82,7 @@ struct Ring {
       tickets->word = nullptr;
     }
     (void)hipHostFree(base);
-    base = nullptr;
-    tickets.reset();
-    head = 0;
-    next = 1;
-    for (auto& q : quarter) q = {};
   }
-  ~Ring() { drop(); }
 };
 thread_local Ring g_ring;
 
@@ -113,10 +105,8 @@ int stage_copy(void* dst, const void* src, size_t bytes, hipStream_t st) {
     return 0;
   }
   Ring& r = g_ring;
-  int dev = 0;
-  TQSV_HIP(hipGetDevice(&dev));
-  if (!r.base || r.dev != dev) {
-    const int rc = r.open(dev);
+  if (!r.base) {
+    const int rc = r.open();
     if (rc) return rc;
   }
   const size_t len = (bytes + 63) & ~(size_t)63;
