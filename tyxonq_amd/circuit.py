@@ -505,6 +505,10 @@ def _as_matrix(m: Any) -> np.ndarray:
 
 
 def _to_numpy(x: Any) -> np.ndarray:
+    if getattr(x, "is_cuda", False):
+        from ._native import to_host
+
+        return to_host(x.detach()).astype(np.complex128)
     if hasattr(x, "detach"):
         return x.detach().cpu().numpy().astype(np.complex128)
     return np.asarray(x, dtype=np.complex128)

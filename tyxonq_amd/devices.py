@@ -171,6 +171,10 @@ def _run_one(eng: Any, device: str, c: Any, shots: int, opts: Dict[str, Any]) ->
     if int(shots) == 0 and not error:
         try:
             psi = _attached_state(eng, c)
+            if getattr(psi, "is_cuda", False):
+                from ._native import to_host
+
+                psi = to_host(psi)
             statevec = (psi.cpu().numpy() if hasattr(psi, "cpu") else np.asarray(psi)
                         ).astype(np.complex128)
             prob = np.abs(statevec) ** 2

@@ -566,7 +566,7 @@ class StatevectorEngine:
         """engine.py:897-1039."""
         psi = self.state_tensor(circuit, mode="state")
         if self.backend.name == "numpy":
-            return psi.detach().cpu().numpy().astype(np.complex128)
+            return nat.to_host(psi.detach()).astype(np.complex128)
         return psi
 
     def run(self, circuit: Any, shots: Optional[int] = None, **kwargs: Any) -> Dict[str, Any]:
@@ -678,7 +678,7 @@ class StatevectorEngine:
                 if nat.norm2(psi) > 0.0:
                     raise
                 # a zero state: the reference draws uniformly (engine.py:409-412)
-        p = nat.probs(psi).cpu().numpy()
+        p = nat.to_host(nat.probs(psi))
         dim = p.size
         if bool(kwargs.get("use_noise", False)):
             noise = kwargs.get("noise", {}) or {}
@@ -788,7 +788,7 @@ class StatevectorEngine:
     def probability(self, circuit: Any) -> np.ndarray:
         """engine.py:1041-1047."""
         psi = self.state_tensor(circuit, mode="state").detach()
-        return nat.probs(psi).cpu().numpy()
+        return nat.to_host(nat.probs(psi))
 
     def amplitude(self, circuit: Any, bitstring: str) -> complex:
         """engine.py:1049-1059 (big-endian: q0 is the leftmost character)."""
