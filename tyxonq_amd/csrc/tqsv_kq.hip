@@ -17,9 +17,9 @@
 // per chunk of 64 columns of U for k >= 7, where each work-group computes 64
 // of the 2^k output rows.
 // Measured per call (one thread per amplitude -> here; random targets): 24
-// qubits, k = 4: 379 -> 58 us, 5: 704 -> 72, 6: 1017 -> 114 (75
-// TFLOP/s with the call, of the 150 a large FP32 matrix product reaches); 27
-// qubits, k = 5: 4.41 -> 0.45 ms (4.8 TB/s); 24 qubits, k = 8: 8.9 -> 0.35 ms.
+// qubits, k = 4: 379 -> 58 us, 5: 704 -> 72, 6: 1124 -> 107 (80 TFLOP/s with the
+// call, of the 150 a large FP32 matrix product reaches); 27 qubits, k = 5: 4.41
+// -> 0.45 ms (4.8 TB/s); 24 qubits, k = 8: 8.9 -> 0.35 ms.
 // Error against 64 bits at k = 6: 1.5e-7 -> 1.1e-7.
 #include <hip/hip_runtime.h>
 

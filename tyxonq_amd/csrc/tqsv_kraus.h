@@ -18,8 +18,9 @@ uint32_t kraus_grid(int n);
 // partials of (rho00, rho11, Re rho01, Im rho01) of the qubit at `bit`
 hipError_t k_kraus_rho(const float2* psi, int n, int bit, double* partials, hipStream_t st);
 // Chooses the item's operator from the sums in `in` (all blocks the same
-// way), applies it, scaled by a power of two to a norm near 1, to `bit`, and writes the partials of the
-// result: of the qubit at `next`, or with next < 0 of the same qubit.
+// way), applies it to `bit`, scaled by a power of two to a norm in [1, 2), and
+// writes the partials of the result: of the qubit at `next`, or with next < 0 of
+// the same qubit.
 hipError_t k_kraus_apply(float2* psi, int n, int bit, int next, const KrausItem* item,
                          const double* ops, const double* in, double* out, hipStream_t st);
 // psi /= sqrt(sum of rho00 + rho11 in `in`) unless that is 0

@@ -5,8 +5,8 @@
 // Tr(K_i^dagger K_i rho), rho the qubit's 2x2 density matrix.  A chain of
 // channels is one sweep per channel: every block sums the partials that the
 // previous sweep left (all in the same order, so all choose alike), applies
-// the chosen operator (times a power of two) to its amplitudes and accumulates the density matrix of
-// the next channel's qubit from the result.  Bound: one read and one write of
+// the chosen operator (times a power of two) to its amplitudes and accumulates
+// the density matrix of the next channel's qubit from the result.  Bound: one read and one write of
 // the state per channel, and launch latency below about 22 qubits.  FP64 sums.
 // 20 qubits, a trajectory of 3 layers with 20 two-operator channels each and
 // <Z> of every qubit: 9.3 ms when every operator was applied to a copy, reduced
@@ -122,9 +122,9 @@ __global__ __launch_bounds__(BLK) void kraus_apply_kernel(float2* __restrict__ p
       }
       const double* k = k0 + 8 * (size_t)sel;
       const double w = weight(k);
-      // the nearest power of two to 1 / sqrt(w): exact, so that the operator's
-      // entries are rounded as they are given, whatever w is; the chain's last
-      // sweep normalises
+      // a power of two, which brings the norm sqrt(w) into [1, 2): exact, so that
+      // the operator's entries are rounded as they are given, whatever w is; the
+      // chain's last sweep normalises
       int x = 0;
       (void)frexp(w, &x);
       const int e2 = w > 0.0 ? -((x - 1) >> 1) : 0;

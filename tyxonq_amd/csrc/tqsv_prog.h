@@ -1,17 +1,19 @@
 // tqsv_prog.h - word layout of the tile-pass programs that the host planner
-// (tqsv_plan.cpp, tqsv_ham.cpp) writes and the pass kernel (tqsv_pass_impl.h)
-// interprets.
+// (tqsv_plan.cpp, tqsv_ham.cpp) writes.  Gate and dual passes are interpreted by
+// tqsv_interp.h, expectation passes by tqsv_pass_impl.h; generated kernels
+// (tqsv_jit.cpp) have the steps compiled in and read only their values.
 //
 // A state of 2^n amplitudes is swept in tiles of 2^T amplitudes.  A tile is
 // the set of amplitudes that agree on every index bit outside the tile's bit
 // set { 0 .. L-1 } U { H[0] .. H[m-1] } (T = L + m).  Tile position p maps to
 // the global index bits as: p bits [0, L) -> index bits [0, L); p bit L+k ->
 // index bit H[k].  A work-group holds one tile in LDS and runs the pass's
-// phases over it; in a phase every thread holds 2^RB amplitudes in registers
-// ("slots") whose tile positions differ only in the RB "register positions"
-// R[0..RB).  Slot s holds the amplitude whose register-position bits equal the
-// bits of s; the other index bits ("thread bits") are fixed per thread and
-// are read from the thread's global index gb (the index of its slot 0).
+// phases over it; in a phase 2^RB amplitudes ("slots") whose tile positions
+// differ only in the RB "register positions" R[0..RB) are held in the registers
+// of one thread, or in tqsv_interp.h of four neighbouring lanes (slot bits 0 and
+// 1 are lane bits there).  Slot s holds the amplitude whose register-position
+// bits equal the bits of s; the other index bits ("thread bits") are fixed per
+// thread (or quad) and are read from its global index gb (the index of slot 0).
 #ifndef TQSV_PROG_H
 #define TQSV_PROG_H
 
@@ -25,7 +27,7 @@ typedef unsigned long long uint64_t;
 namespace tqsv {
 
 constexpr int RB = 5;              // register bits per phase
-constexpr int NSLOT = 1 << RB;     // amplitudes per thread per state
+constexpr int NSLOT = 1 << RB;     // slots of a phase, per state
 constexpr int MAXH = 9;            // maximum number of non-contiguous tile bits
 
 // pass flags
