@@ -174,9 +174,10 @@ def _run_one(eng: Any, device: str, c: Any, shots: int, opts: Dict[str, Any]) ->
             if getattr(psi, "is_cuda", False):
                 from ._native import to_host
 
-                psi = to_host(psi)
-            statevec = (psi.cpu().numpy() if hasattr(psi, "cpu") else np.asarray(psi)
-                        ).astype(np.complex128)
+                host = to_host(psi)
+            else:
+                host = psi.cpu().numpy() if hasattr(psi, "cpu") else np.asarray(psi)
+            statevec = host.astype(np.complex128)
             prob = np.abs(statevec) ** 2
             meta.setdefault("num_qubits", int(getattr(c, "num_qubits", 0)))
         except Exception as e:
