@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <new>
 #include <vector>
@@ -698,17 +699,20 @@ int tqsv_sampler_run(tqsv_sampler* s, const void* psi, int64_t shots, uint64_t s
     // shots from 26 qubits, dense and of two basis states: with a round trip 400 and
     // 5130 us, with every entry that there could be (1.6 MB) 316 and 5130, so 300
     // and 5060
-    for (uint32_t k = 1; __atomic_load_n(&s->head->call, __ATOMIC_ACQUIRE) != s->calls; ++k)
-      if (k % 4096u == 0) {
-        const hipError_t q = hipStreamQuery(st);
-        if (q == hipErrorNotReady) {
-          (void)hipGetLastError();
-          continue;
-        }
+    // (a query of the stream, for a launch that failed, costs the device a packet:
+    // every 20 ms)
+    auto ask = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
+    for (uint32_t k = 1; __atomic_load_n(&s->head->call, __ATOMIC_ACQUIRE) != s->calls; ++k) {
+      if (k % 4096u != 0 || std::chrono::steady_clock::now() < ask) continue;
+      const hipError_t q = hipStreamQuery(st);
+      if (q != hipErrorNotReady) {
         TQSV_HIP(q);
         if (__atomic_load_n(&s->head->call, __ATOMIC_ACQUIRE) != s->calls)
           return fail(TQSV_EDEVICE, "tqsv_sampler_run: no result");
       }
+      (void)hipGetLastError();
+      ask = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
+    }
     const uint64_t most = std::min<uint64_t>(ns, s->n < 32 ? 1ull << s->n : ns);
     const double total = s->head->total;
     const uint64_t nu = s->head->nuniq;
